@@ -58,7 +58,21 @@ constexpr int kGgPairRoutes = 64;                  // routes per work item of by
 constexpr int kGgWaveTiles = 4;                    // 16-row weight tiles per wave
 constexpr int kGgRows = kGgWaves * kGgWaveTiles * 16;  // 256 weight rows per workgroup
 constexpr int kGgStride = kGroup + 16;             // LDS bytes per staged route row
+constexpr int kGgRowF = kGgRows + 4;               // floats per route row of FC2's epilogue buffers
+static_assert(2 * 16 * kGgRowF * 4 <= 2 * kGgRoutes * kGgStride, "two epilogue buffers fit the staging ring");
 constexpr int kGgXcds = 8;
+// Launches whose experts average at most this many routes at capacity run
+// the sparse kernel, if they fill a round of resident workgroups (two per
+// CU): below one round the launch is a single prologue and K loop, which the
+// 128-route kernel runs 0.5 us faster (E16 H1024 I256, 140 rows: FC1 15.7
+// against 16.1 us).  Kernel trace, FC1 / FC2 us, 128-route kernel -> sparse:
+// E256 I512 3,000 rows (94 routes per expert) 119.5 / 95.7 -> 114.5 / 88.0,
+// 3,300 rows (103) 123.3 / 98.5 -> 120.2 / 93.6, 3,600 rows (113) 137.3 /
+// 100.9 -> 138.5 / 98.7; E128 I768 1,500 rows (94) 96.6 / 64.3 -> 92.0 / 62.0,
+// 1,700 rows (106) 97.5 / 71.1 -> 98.1 / 71.5, 1,900 rows (119) 99.7 / 71.6
+// -> 110.6 / 77.4.
+constexpr int kSparseRoutes = 104;
+constexpr int kResidentGroups = 512;
 constexpr int kStreamOutRoutes = 16384;  // FC2 launches up to this many item routes stream their rows
 // Routes found by the workgroups themselves (by-pair launches): at most this
 // many (row, rank) pairs, read in chunks of one id per thread.
@@ -77,6 +91,84 @@ struct SharedItems {
   int pos;
   int pair;
 };
+
+// FC2 epilogue: each route tile's 16 x 256 fp32 block goes through LDS (two
+// buffers in `tbuf`) so that every store writes one route's 1 KiB run.
+template <int kRT, bool kStreamOut>
+__device__ __forceinline__ void store_fc2(const floatx4 (&acc)[kGgWaveTiles][kRT], const int* target, float* tbuf,
+                                          int n_rows, int n0, int lane, int wave, int row16, int group,
+                                          float* __restrict__ out_f32) {
+#pragma unroll
+  for (int rt = 0; rt < kRT; ++rt) {
+    float* buf = tbuf + (rt & 1) * 16 * kGgRowF;
+#pragma unroll
+    for (int t = 0; t < kGgWaveTiles; ++t)
+      *reinterpret_cast<floatx4*>(buf + row16 * kGgRowF + 64 * wave + 16 * t + 4 * group) = acc[t][rt];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = 4 * wave + j;
+      const int pair = target[16 * rt + r];
+      const floatx4 v = *reinterpret_cast<const floatx4*>(buf + r * kGgRowF + 4 * lane);
+      if (pair >= 0) {
+        float* dst = out_f32 + static_cast<size_t>(pair) * n_rows + n0 + 4 * lane;
+        if constexpr (kStreamOut)
+          __builtin_nontemporal_store(v, reinterpret_cast<floatx4*>(dst));
+        else
+          *reinterpret_cast<floatx4*>(dst) = v;
+      }
+    }
+  }
+}
+
+// FC1 epilogue: SwiGLU on the bf16-rounded FC1 outputs, the per-(route,
+// 128-column) amax across lanes and waves, e4m3 codes and scales.
+template <int kRT, int kR>
+__device__ __forceinline__ void store_fc1(const floatx4 (&acc)[kGgWaveTiles][kRT], const int* target,
+                                          float (&amax_part)[kGgWaves][kR], int out_cols, int n0, int tile, int wave, int row16,
+                                          int group, uint8_t* __restrict__ out_codes, float* __restrict__ out_scales) {
+  // Lane holds gate / up columns
+  // 32 wave + 16 p + 4 group + i (p < 2, i < 4) of route 16 rt + row16.
+  float v[kRT][8];
+#pragma unroll
+  for (int rt = 0; rt < kRT; ++rt) {
+    float g[8], u[8];
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        const uint32_t gw = pack_bf16x2(acc[p][rt][i], acc[p][rt][i + 1]);
+        const uint32_t uw = pack_bf16x2(acc[2 + p][rt][i], acc[2 + p][rt][i + 1]);
+        g[4 * p + i] = bf16_lo(gw);
+        g[4 * p + i + 1] = bf16_hi(gw);
+        u[4 * p + i] = bf16_lo(uw);
+        u[4 * p + i + 1] = bf16_hi(uw);
+      }
+    swiglu_values<8>(g, u, v[rt]);
+    float amax = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[rt][k]));
+    amax = fmaxf(amax, __shfl_xor(amax, 16));
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    if (group == 0) amax_part[wave][16 * rt + row16] = amax;
+  }
+  __syncthreads();
+  const int groups = out_cols / kGroup;
+#pragma unroll
+  for (int rt = 0; rt < kRT; ++rt) {
+    const int route = 16 * rt + row16;
+    const int position = target[route];
+    if (position < 0) continue;
+    float amax = amax_part[0][route];
+#pragma unroll
+    for (int q = 1; q < kGgWaves; ++q) amax = fmaxf(amax, amax_part[q][route]);
+    const float scale = group_scale(amax);
+    uint8_t* dst = out_codes + static_cast<size_t>(position) * out_cols + n0 + 32 * wave + 4 * group;
+    *reinterpret_cast<uint32_t*>(dst) = quantize_four(&v[rt][0], scale);
+    *reinterpret_cast<uint32_t*>(dst + 16) = quantize_four(&v[rt][4], scale);
+    if (wave == 0 && group == 0) out_scales[static_cast<size_t>(position) * groups + tile] = scale;
+  }
+}
 
 // kByPair (FC1 of small batches): no sorted route list.  A work item is
 // part j (routes [64 j, 64 j + 64) in pair order) of an expert; the
@@ -416,76 +508,273 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
     __syncthreads();
   }
 
-  if constexpr (MODE == 1) {
-    // Each route tile's 16 x 256 fp32 block goes through LDS (two buffers in
-    // the staging ring) so that every store writes one route's 1 KiB run.
-    constexpr int kRowF = kGgRows + 4;
-    static_assert(2 * 16 * kRowF * 4 <= 2 * kStage, "epilogue buffers fit the staging ring");
-    float* tbuf = reinterpret_cast<float*>(&stage[0][0]);
+  if constexpr (MODE == 1)
+    store_fc2<kRT, kStreamOut>(acc, target, reinterpret_cast<float*>(&stage[0][0]), n_rows, n0, lane, wave, row16, group, out_f32);
+  else
+    store_fc1<kRT>(acc, target, amax_part, out_cols, n0, tile, wave, row16, group, out_codes, out_scales);
+}
+
+// Launches that stream more weights than they compute (few routes per
+// expert): see grouped_sparse_kernel.
+struct SparseArgs {
+  const uint8_t* w;
+  const float* ws;
+  int n_rows, out_cols;
+  const uint8_t* act;
+  uint32_t act_bytes;
+  const float* act_scales;
+  const int32_t* sorted_ids;
+  int top_k;
+  const int4* items;
+  const int32_t* num_items;
+  int max_items;
+  SharedItems shared;
+  int n_tiles, chunk;
+  uint8_t* out_codes;
+  float* out_scales;
+  float* out_f32;
+};
+
+// One workgroup's work, all wave-uniform.
+struct SparseItem {
+  const uint8_t* w;  // the expert's weights and block scales
+  const float* ws;
+  int first, routes, tile;
+  bool dense;  // shared-expert rows
+};
+
+template <int KB, int MODE>
+struct SparseLds {
+  __attribute__((aligned(16))) uint8_t stage[2][kGgRoutes * kGgStride];
+  float a_scale[KB][kGgRoutes];
+  int target[kGgRoutes];  // FC1: sorted position, FC2: pair; -1 = no route
+  float amax_part[MODE == 0 ? kGgWaves : 1][kGgRoutes];
+};
+
+// One work item of the sparse kernel at kRT 16-route tiles (routes <= 16
+// kRT).  kDepth K blocks of weights are in flight (each reloads the
+// registers of the block just multiplied), and as many of staged activations
+// (one for kRT > 4, whose accumulators need the registers).  The MFMAs, the
+// scale products and their order are those of grouped_gemm_kernel, so the
+// results are bit-identical.
+template <int KB, int MODE, bool kPacked, bool kStreamOut, int kRT, int kDepth>
+__device__ __forceinline__ void sparse_item(const SparseArgs& a, const SparseItem& item,
+                                            SparseLds<KB, MODE>& lds) {
+  constexpr int K = KB * kGroup;
+  constexpr int kR = 16 * kRT;
+  constexpr int kStage = kR * kGgStride;
+  constexpr int kD = kDepth < KB ? kDepth : KB;             // K blocks in flight
+  constexpr int kA = kRT > 4 ? 1 : kD;                       // K blocks of activations in registers
+  constexpr int kStaged = kR * kGroup / (16 * kGgThreads);  // 16-byte copies per thread and K block
+  static_assert(kStaged >= 1, "at least 32 routes: one copy per thread and K block");
+  const int n_rows = a.n_rows, out_cols = a.out_cols, top_k = a.top_k;
+  const int first = item.first, routes = item.routes, tile = item.tile;
+  const bool dense = item.dense;
+  const uint8_t* __restrict__ wexp = item.w;
+  const float* __restrict__ wsexp = item.ws;
+  uint8_t* stage = &lds.stage[0][0];
+  const int tid = threadIdx.x;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int row16 = lane & 15;
+  const int group = lane >> 4;
+  const int n0 = tile * (MODE == 0 ? kGroup : kGgRows);
+  auto tile_row = [&](int t) {
+    if constexpr (MODE == 0)
+      return (t < 2 ? 0 : out_cols) + n0 + 32 * wave + 16 * (t & 1);
+    else
+      return n0 + 64 * wave + 16 * t;
+  };
+  // Route ids first: the loads that depend on them come back after the first
+  // weights, and waiting for the ids does not cover any weight.
+  const int part = tid & 7;
+  const int r0 = tid >> 3;
+  int ids[kStaged];
 #pragma unroll
-    for (int rt = 0; rt < kRT; ++rt) {
-      float* buf = tbuf + (rt & 1) * 16 * kRowF;
+  for (int i = 0; i < kStaged; ++i) {
+    const int r = r0 + (kGgThreads / 8) * i;
+    ids[i] = dense ? 0 : a.sorted_ids[first + (r < routes ? r : 0)];
+  }
+  constexpr int kRs = kR == 96 ? 128 : kR;  // a power of two
+  const int rs = tid % kRs;
+  const int k0 = tid / kRs;
+  const int id_s = dense ? 0 : a.sorted_ids[first + (rs < routes ? rs : 0)];
+  // Activation row of route r: FC1 the token of its pair, FC2 the sorted
+  // position; shared-expert items map route r to row first + r.
+  const int row0 = MODE == 1 && dense ? a.shared.pos + first : first;
+  auto act_row = [&](int r, int id) { return MODE == 0 && !dense ? id / top_k : row0 + r; };
+  __builtin_amdgcn_sched_barrier(0);
+
+  const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(wexp), 0, static_cast<uint32_t>(n_rows) * K, 0x00020000);
+  const uint32_t w_lane = kPacked ? lane * 16 : row16 * K + group * 16;
+  int32x8 wf[kD][kGgWaveTiles];
+  constexpr int kStreamed = kPacked ? 2 : 0;  // non-temporal: most experts have this item only
+  auto load_weights = [&](int kb) {
 #pragma unroll
-      for (int t = 0; t < kGgWaveTiles; ++t)
-        *reinterpret_cast<floatx4*>(buf + row16 * kRowF + 64 * wave + 16 * t + 4 * group) = acc[t][rt];
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = 4 * wave + j;
-        const int pair = target[16 * rt + r];
-        const floatx4 v = *reinterpret_cast<const floatx4*>(buf + r * kRowF + 4 * lane);
-        if (pair >= 0) {
-          float* dst = out_f32 + static_cast<size_t>(pair) * n_rows + n0 + 4 * lane;
-          if constexpr (kStreamOut)
-            __builtin_nontemporal_store(v, reinterpret_cast<floatx4*>(dst));
-          else
-            *reinterpret_cast<floatx4*>(dst) = v;
-        }
+    for (int t = 0; t < kGgWaveTiles; ++t) {
+      const uint32_t base = static_cast<uint32_t>(tile_row(t)) * K;
+      int32x4 lo, hi;
+      if constexpr (kPacked) {
+        lo = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * 2048, kStreamed);
+        hi = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * 2048 + 1024, kStreamed);
+      } else {
+        lo = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * kGroup, kStreamed);
+        hi = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * kGroup + 64, kStreamed);
       }
+      int32x8 v;
+      v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
+      v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
+      wf[kb % kD][t] = v;
     }
-  } else {
-    // SwiGLU on the bf16-rounded FC1 outputs; lane holds gate / up columns
-    // 32 wave + 16 p + 4 group + i (p < 2, i < 4) of route 16 rt + row16.
-    float v[kRT][8];
+  };
+  constexpr int kEarly = (kD + 1) / 2;  // weight blocks issued before the activations
 #pragma unroll
-    for (int rt = 0; rt < kRT; ++rt) {
-      float g[8], u[8];
+  for (int kb = 0; kb < kEarly; ++kb) load_weights(kb);
+  __builtin_amdgcn_sched_barrier(0);
+
+  const BufferView view(a.act, a.act_bytes);
+  uint32_t src[kStaged];
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
+  for (int i = 0; i < kStaged; ++i) {
+    const int r = r0 + (kGgThreads / 8) * i;
+    src[i] = r < routes ? static_cast<uint32_t>(act_row(r, ids[i])) * K + part * 16 : kNoRow;
+  }
+  int4 staged[kA][kStaged];
+  auto stage_load = [&](int kb) {
 #pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-          const uint32_t gw = pack_bf16x2(acc[p][rt][i], acc[p][rt][i + 1]);
-          const uint32_t uw = pack_bf16x2(acc[2 + p][rt][i], acc[2 + p][rt][i + 1]);
-          g[4 * p + i] = bf16_lo(gw);
-          g[4 * p + i + 1] = bf16_hi(gw);
-          u[4 * p + i] = bf16_lo(uw);
-          u[4 * p + i + 1] = bf16_hi(uw);
-        }
-      swiglu_values<8>(g, u, v[rt]);
-      float amax = 0.0f;
+    for (int i = 0; i < kStaged; ++i) staged[kb % kA][i] = view.load16(src[i] + kb * kGroup);
+  };
+  auto stage_store = [&](int kb) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[rt][k]));
-      amax = fmaxf(amax, __shfl_xor(amax, 16));
-      amax = fmaxf(amax, __shfl_xor(amax, 32));
-      if (group == 0) amax_part[wave][16 * rt + row16] = amax;
+    for (int i = 0; i < kStaged; ++i)
+      *reinterpret_cast<int4*>(stage + (kb & 1) * kStage + (r0 + (kGgThreads / 8) * i) * kGgStride + part * 16) =
+          staged[kb % kA][i];
+  };
+#pragma unroll
+  for (int kb = 0; kb < kA; ++kb) stage_load(kb);
+  constexpr int kSplit = kGgThreads / kRs;  // threads per route row of scales
+  const bool live = rs < routes;
+  float sc[(KB + kSplit - 1) / kSplit];
+  {
+    const float* srow = a.act_scales + static_cast<size_t>(act_row(live ? rs : 0, id_s)) * KB;
+#pragma unroll
+    for (int q = 0; q < (KB + kSplit - 1) / kSplit; ++q) sc[q] = srow[min(q * kSplit + k0, KB - 1)];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int kb = kEarly; kb < kD; ++kb) load_weights(kb);
+  float w_rows[2][KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    w_rows[0][kb] = wsexp[(tile_row(0) / kGroup) * KB + kb];
+    w_rows[1][kb] = wsexp[(tile_row(2) / kGroup) * KB + kb];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < (KB + kSplit - 1) / kSplit; ++q)
+    if (q * kSplit + k0 < KB) lds.a_scale[q * kSplit + k0][rs] = live ? sc[q] : 0.0f;
+  int out_row = MODE == 1 ? id_s : first + rs;
+  if (dense) out_row = (MODE == 0 ? a.shared.pos : a.shared.pair) + first + rs;
+  if (k0 == 0) lds.target[rs] = live ? out_row : -1;
+  stage_store(0);
+  lds_barrier();
+
+  floatx4 acc[kGgWaveTiles][kRT];
+#pragma unroll
+  for (int t = 0; t < kGgWaveTiles; ++t)
+#pragma unroll
+    for (int rt = 0; rt < kRT; ++rt) acc[t][rt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kA == 1) {
+      if (kb + 1 < KB) stage_load(kb + 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-    const int groups = out_cols / kGroup;
+    const uint8_t* buf = stage + (kb & 1) * kStage;
 #pragma unroll
     for (int rt = 0; rt < kRT; ++rt) {
       const int route = 16 * rt + row16;
-      const int position = target[route];
-      if (position < 0) continue;
-      float amax = amax_part[0][route];
+      const int32x8 bfrag = load_fragment(buf + route * kGgStride, 0, group);
+      const float as = lds.a_scale[kb][route];
 #pragma unroll
-      for (int q = 1; q < kGgWaves; ++q) amax = fmaxf(amax, amax_part[q][route]);
-      const float scale = group_scale(amax);
-      uint8_t* dst = out_codes + static_cast<size_t>(position) * out_cols + n0 + 32 * wave + 4 * group;
-      *reinterpret_cast<uint32_t*>(dst) = quantize_four(&v[rt][0], scale);
-      *reinterpret_cast<uint32_t*>(dst + 16) = quantize_four(&v[rt][4], scale);
-      if (wave == 0 && group == 0) out_scales[static_cast<size_t>(position) * groups + tile] = scale;
+      for (int t = 0; t < kGgWaveTiles; ++t) {
+        const floatx4 partial = mfma_fp8(wf[kb % kD][t], bfrag);
+        scale_accumulate(acc[t][rt], partial, w_rows[t < 2 ? 0 : 1][kb] * as);
+        asm volatile("" : "+v"(acc[t][rt]));
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if (kb + kD < KB) {  // into the registers this block has just left
+      if constexpr (kA > 1) stage_load(kb + kD);
+      load_weights(kb + kD);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (kb + 1 < KB) stage_store(kb + 1);
+    lds_barrier();
   }
+
+
+  if constexpr (MODE == 1)
+    store_fc2<kRT, kStreamOut>(acc, lds.target, reinterpret_cast<float*>(stage), n_rows, n0, lane, wave, row16, group, a.out_f32);
+  else
+    store_fc1<kRT>(acc, lds.target, lds.amax_part, out_cols, n0, tile, wave, row16, group, a.out_codes, a.out_scales);
+}
+
+// The GEMMs of sparse batches (at most kSparseRoutes routes per expert on
+// average): bound by the weight stream, each expert's weights being read
+// once, by its one work item.  grouped_gemm_kernel spends its registers on
+// 128 accumulators and has one K block in flight; here the workgroup picks
+// the smallest of four bodies that holds its item (32, 64, 96 or 128 routes)
+// and the registers go to weights in flight, read non-temporally.  Measured
+// (E256 H2048 I512, FC1 / FC2 us, kernel trace, one box): 131 rows (4 routes
+// per expert) 104.8 / 61.8 -> 87.6 / 46.1 (6.1 / 6.0 TB/s), 517 rows of an
+// uneven router 92.0 / 60.2 -> 84.1 / 48.4, 2048 rows (64 per expert) 117.3 /
+// 84.0 -> 106.6 / 78.6; non-temporal loads are half of the gain.  Two more
+// depths were tried (2 and 4 to 5 blocks for the 32-route body): within 1 us,
+// 5 spills.  At 128 routes per expert (4,096 rows) it is slower (144 / 118 ->
+// 152 / 118 us cached, 165 / 126 us non-temporal): the matrix work then wants
+// the loads spread between the MFMAs and the experts' second items the
+// weights in L2.
+template <int KB, int MODE, bool kPacked, bool kStreamOut>
+__global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2))) void grouped_sparse_kernel(
+    SparseArgs a) {
+  constexpr int K = KB * kGroup;
+  __shared__ SparseLds<KB, MODE> lds;
+  // Workgroups to (item, tile) as in grouped_gemm_kernel.
+  const int b = blockIdx.x;
+  const int xcd = b % kGgXcds, j = b / kGgXcds;
+  const int logical = ((j / a.chunk) * kGgXcds + xcd) * a.chunk + j % a.chunk;
+  const int within = logical % a.chunk;
+  const int item_index = (logical / a.chunk) * 2 + (within & 1);
+  SparseItem item;
+  item.tile = within >> 1;
+  item.dense = item_index >= a.max_items;
+  if (!item.dense) {
+    // both loads in flight together, one exit
+    const int4 entry = a.items[item_index];
+    const int count = *a.num_items;
+    item.first = entry.y;
+    item.routes = item_index < count ? min(entry.z, kGgRoutes) : 0;
+    if (item.routes <= 0) return;  // a padding item (uniform)
+    item.w = a.w + static_cast<size_t>(entry.x) * a.n_rows * K;
+    item.ws = a.ws + static_cast<size_t>(entry.x) * (a.n_rows / kGroup) * KB;
+  } else {
+    item.first = (item_index - a.max_items) * kGgRoutes;
+    if (item.first >= a.shared.rows) return;
+    item.routes = min(kGgRoutes, a.shared.rows - item.first);
+    item.w = a.shared.w;
+    item.ws = a.shared.ws;
+  }
+  if (item.routes <= 32)
+    sparse_item<KB, MODE, kPacked, kStreamOut, 2, 3>(a, item, lds);
+  else if (item.routes <= 64)
+    sparse_item<KB, MODE, kPacked, kStreamOut, 4, 3>(a, item, lds);
+  else if (item.routes <= 96)
+    sparse_item<KB, MODE, kPacked, kStreamOut, 6, 2>(a, item, lds);
+  else
+    sparse_item<KB, MODE, kPacked, kStreamOut, 8, 2>(a, item, lds);
 }
 
 struct GroupedLaunch {
@@ -513,6 +802,7 @@ struct GroupedLaunch {
   int32_t* list_ids = nullptr;  // by-pair launches: the route list they write
   int4* list_items = nullptr;
   int32_t* list_count = nullptr;
+  bool sparse = false;  // few routes per expert (kSparseRoutes)
 };
 
 template <int KB, int MODE>
@@ -524,6 +814,30 @@ void launch_grouped(const GroupedLaunch& g, hipStream_t s) {
   const int64_t logical = (static_cast<int64_t>(g.max_items) + shared_items) * n_tiles;
   const int64_t per_round = static_cast<int64_t>(kGgXcds) * chunk;
   const int blocks = static_cast<int>((logical + per_round - 1) / per_round * per_round);
+  // FC2 rows of small batches (the mixed step's few thousand routes) go out
+  // with non-temporal stores: measured 1.4 us less per mixed step, while the
+  // prefill batch (29k routes, 240 MB of rows) is 10 us slower that way.
+  const bool stream_out =
+      MODE == 1 && (static_cast<int64_t>(g.max_items) + shared_items) * kGgRoutes <= kStreamOutRoutes;
+  if (g.sparse && logical >= kResidentGroups) {
+    const SparseArgs a{g.w, g.ws, g.n_rows, g.out_cols, g.a, g.a_bytes, g.as, g.sorted_ids, g.top_k, g.items,
+                       g.num_items, g.max_items, g.shared, n_tiles, chunk, g.codes, g.scales, g.out};
+    const bool packed = g.layout == D3_LAYOUT_FRAGMENT;
+    if constexpr (MODE == 1) {
+      if (stream_out) {
+        if (packed)
+          hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, true, true>), dim3(blocks), dim3(kGgThreads), 0, s, a);
+        else
+          hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, false, true>), dim3(blocks), dim3(kGgThreads), 0, s, a);
+        return;
+      }
+    }
+    if (packed)
+      hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, true, false>), dim3(blocks), dim3(kGgThreads), 0, s, a);
+    else
+      hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, false, false>), dim3(blocks), dim3(kGgThreads), 0, s, a);
+    return;
+  }
 #define D3_GG_ARGS dim3(blocks), dim3(kGgThreads), 0, s, g.w, g.ws, g.n_rows, g.out_cols, g.a, \
                    g.a_bytes, g.as, g.sorted_ids, g.top_k, g.items, g.num_items, g.max_items, \
                    g.shared, n_tiles, chunk, g.parts, g.capacity, g.list_ids, g.list_items,   \
@@ -538,10 +852,7 @@ void launch_grouped(const GroupedLaunch& g, hipStream_t s) {
     }
   }
   if constexpr (MODE == 1) {
-    // Small batches (the mixed step's few thousand routes) write FC2's fp32
-    // rows non-temporally: measured 1.4 us less per mixed step, while the
-    // prefill batch (29k routes, 240 MB of rows) is 10 us slower that way.
-    if ((static_cast<int64_t>(g.max_items) + shared_items) * kGgRoutes <= kStreamOutRoutes) {
+    if (stream_out) {
       if (g.layout == D3_LAYOUT_FRAGMENT)
         hipLaunchKernelGGL((grouped_gemm_kernel<KB, MODE, true, false, true>), D3_GG_ARGS);
       else
@@ -611,11 +922,12 @@ extern "C" int d3_grouped_fc1_swiglu(const uint8_t* w13, const float* s13, int32
   D3_REQUIRE(intermediate > 0 && intermediate % kGroup == 0,
              "grouped_fc1_swiglu: intermediate %d must be a multiple of 128", intermediate);
   D3_REQUIRE(aligned_to(act, 4), "grouped_fc1_swiglu: act must be 4-byte aligned");
-  const GroupedLaunch g{0, weight_layout, w13, s13, 2 * intermediate, intermediate, q,
+  GroupedLaunch g{0, weight_layout, w13, s13, 2 * intermediate, intermediate, q,
                         static_cast<uint32_t>(q_rows * hidden), x_scales, sorted_ids, top_k,
                         reinterpret_cast<const int4*>(items), num_items, max_items, item_rows,
                         SharedItems{shared_w13, shared_s13, shared_rows, shared_act_row, 0}, act,
                         act_scales, nullptr};
+  g.sparse = q_rows * top_k <= static_cast<int64_t>(kSparseRoutes) * num_experts;
   int status = check_grouped(g, num_experts, hidden, q_rows, "grouped_fc1_swiglu");
   if (status != D3_OK) return status;
   if (max_items == 0 && !(shared_w13 && shared_rows > 0)) {
@@ -644,11 +956,14 @@ extern "C" int d3_grouped_fc2(const uint8_t* w2, const float* s2, int32_t weight
   D3_SUPPORTED(hidden > 0 && hidden % kGgRows == 0,
                "grouped_fc2: hidden %d must be a multiple of %d", hidden, kGgRows);
   D3_REQUIRE(aligned_to(down, 16), "grouped_fc2: down must be 16-byte aligned");
-  const GroupedLaunch g{1, weight_layout, w2, s2, hidden, hidden, act,
+  GroupedLaunch g{1, weight_layout, w2, s2, hidden, hidden, act,
                         static_cast<uint32_t>(act_rows * intermediate), act_scales, sorted_ids, top_k,
                         reinterpret_cast<const int4*>(items), num_items, max_items, item_rows,
                         SharedItems{shared_w2, shared_s2, shared_rows, shared_act_row, shared_out_row},
                         nullptr, nullptr, down};
+  // The sorted rows hold the pairs and up to 15 padding rows per expert (at
+  // the 16-row sort tile; wider tiles and by-pair lists never come this low).
+  g.sparse = act_rows - shared_rows <= static_cast<int64_t>(kSparseRoutes + 16) * num_experts;
   int status = check_grouped(g, num_experts, intermediate, act_rows, "grouped_fc2");
   if (status != D3_OK) return status;
   if (max_items == 0 && !(shared_w2 && shared_rows > 0)) {

@@ -76,6 +76,77 @@ def test_grouped_matches_fp8_chain(device, shape, packed, item_rows):
     assert torch.equal(ws.down.view(torch.int32), down_ref.view(torch.int32)), "down rows differ"
 
 
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("shape", [(128, 2048, 512), (256, 512, 768), (256, 1024, 256)],
+                         ids=["h2048_i512", "h512_i768", "h1024_i256"])
+def test_grouped_sparse_items_match_fp8_chain(device, shape, packed):
+    """Few routes per expert on average (the launches that pick a body per
+    item): items at both sides of every body's edge, up to two items per
+    expert, byte for byte the FP8 chain's."""
+    from drama3_amd.expert_weights import prepare_experts
+    from drama3_amd.pipeline import MoEWorkspace, Shape
+
+    e, h, i = shape
+    edges = [0, 1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 200, 256]
+    counts = np.full(e, 5)
+    counts[:len(edges)] = edges
+    counts[-1] += -counts.sum() % 8
+    flat = np.repeat(np.arange(e), counts)
+    rows = flat.size // 8
+    assert rows * 8 <= 104 * e and rows > 128  # average at capacity
+    ids = torch.from_numpy(flat.reshape(8, rows).T.copy()).to(device=device, dtype=torch.int32)
+    w, x, _ = _workload(rows, e, h, i, seed=23)
+    experts = w.to(device)
+    if packed:
+        prepare_experts(experts)
+    ws = MoEWorkspace(Shape(rows, e, h, i), device, grouped=True)
+    assert ws.max_items * min(i // 128, h // 256) >= 512  # a full round of workgroups
+    ws.quantize(x.to(device))
+    ws.sort(ids)
+    live = _live_positions(ws)
+    ws.exact_routes = 0
+    ws.fc1(experts)
+    ws.activation()
+    ws.fc2(experts)
+    torch.cuda.synchronize()
+    act_ref, scales_ref, down_ref = ws.act[live].clone(), ws.act_scales[live].clone(), ws.down.clone()
+    ws.act.zero_()
+    ws.act_scales.zero_()
+    ws.down.zero_()
+    ws.grouped_fc1(experts)
+    ws.grouped_fc2(experts)
+    torch.cuda.synchronize()
+    assert torch.equal(ws.act[live], act_ref)
+    assert torch.equal(ws.act_scales[live].view(torch.int32), scales_ref.view(torch.int32))
+    assert torch.equal(ws.down.view(torch.int32), down_ref.view(torch.int32))
+
+
+@pytest.mark.parametrize("rows", [131, 700])
+def test_grouped_sparse_shared_expert(device, rows):
+    """The folded shared expert in a sparse launch: routed rows as without
+    it, shared rows as the dense expert's own launches give them."""
+    from drama3_amd.pipeline import DenseExpert, MoEWorkspace, Shape
+
+    e, h, i = 128, 2048, 512
+    w, x, logits = _workload(rows, e, h, i, seed=29)
+    s, _, _ = _workload(rows, 1, h, i, seed=30)
+    experts, shared = w.to(device), s.to(device)
+    x, logits = x.to(device), logits.to(device)
+    plain = MoEWorkspace(Shape(rows, e, h, i), device)
+    plain.front(x, logits)
+    plain.grouped_fc1(experts)
+    plain.grouped_fc2(experts)
+    folded = MoEWorkspace(Shape(rows, e, h, i), device, shared_rows=rows)
+    folded.front(x, logits)
+    folded.grouped_fc1(experts, shared)
+    folded.grouped_fc2(experts, shared)
+    dense = DenseExpert(rows, h, i, device).forward(folded.q, folded.x_scales, shared)
+    torch.cuda.synchronize()
+    pairs = plain.shape.pairs
+    assert torch.equal(folded.down[:pairs].view(torch.int32), plain.down.view(torch.int32))
+    assert torch.equal(folded.shared_down.view(torch.int32), dense.view(torch.int32))
+
+
 @pytest.mark.parametrize("shape", [(300, 8, 512, 512), (260, 8, 1536, 256), (400, 16, 256, 1536)],
                          ids=["h512_i512", "h1536_i256", "h256_i1536"])
 def test_grouped_other_contraction_lengths(device, shape):
