@@ -18,7 +18,12 @@
 //
 // A workgroup whose expert receives no route exits after its first weight
 // loads (those bytes are wasted): the layout suits batches whose routes
-// cover most experts; sparse ones are better served by the sorted chain.
+// cover most experts.  A handful of rows over many experts (fewer routes
+// than experts, at most 256) takes the pair grid instead: a workgroup per
+// (pair, row tile), whose expert is the pair's; it goes on only if no
+// earlier pair names that expert, and then takes all of the expert's pairs.
+// Every wave holds all the ids (four per lane), so that is decided from four
+// ballots without LDS, and no weight is issued for an expert without routes.
 //
 // The FC1 can also start from the slots themselves (MODE 1), which removes
 // the front launch: slot s routes to expert e at rank c when c, the number
@@ -40,6 +45,7 @@ namespace d3 {
 namespace {
 
 constexpr int kMaxSlots = 256;                        // rows per launch (one route per row and expert)
+constexpr int kPairGridPairs = 256;                   // most pairs of a pair-grid launch
 constexpr int kMaxIds = kMaxSlots * 8;                // ids read per workgroup (top_k <= 8)
 constexpr int kIdsPerThread = kMaxIds / kGemmThreads;  // 8
 
@@ -50,8 +56,11 @@ struct DecodeArgs {
   int capacity;  // slot rows
   int top_k;
   int exact_routes;
-  // MODE 0 / 2: routed ids of every row and the live row count (front output)
+  // MODE 0 / 2 / 3: routed ids of every row (32-bit words, id_words apart)
+  // and the live row count (front output, or none)
   const int32_t* ids;
+  int id_words;
+  int row_routes;  // most routes of one expert in a row: 1 (router ids) or top_k (given ids)
   const int32_t* row_count;
   // MODE 0: q rows and their scales; MODE 2: bf16 gate|up by pair
   const void* act;
@@ -94,6 +103,9 @@ struct LogitPass {
 //         quantised while staged -> bf16 gate|up by pair, ids, count, slots.
 // MODE 2: FC2 with the SwiGLU requant in the prologue, gate|up by pair x W2
 //         -> fp32 down by pair.
+// MODE 3: FC1 from given ids: x rows quantised while staged (as MODE 1) ->
+//         bf16 gate|up by pair.
+// kPairGrid (MODE 0, 2, 3): workgroups by (pair, weight tile).
 // TILES weight tiles per workgroup, streamed through the registers in halves
 // (TILES > 1: routes beyond the first 16 reload the weight tiles).
 // PASSES (MODE 1): ranking passes of 64 slots the kernel is built for.
@@ -103,7 +115,8 @@ struct LogitPass {
 // Launches that may split an expert's route tiles over several workgroups
 // (route slices): one weight tile per workgroup, except FC1 from the slots
 // at K = 2048, whose two bodies together would not fit the registers.
-constexpr bool sliced_kernel(int kb, int mode, int tiles) { return tiles == 1 && !(mode == 1 && kb >= 16); }
+constexpr bool from_x(int mode) { return mode == 1 || mode == 3; }  // FC1 quantises the x rows itself
+constexpr bool sliced_kernel(int kb, int mode, int tiles) { return tiles == 1 && !(from_x(mode) && kb >= 16); }
 
 // LDS of one decode GEMM workgroup (declared once in the kernel, shared by
 // both instantiations of its body).
@@ -114,7 +127,7 @@ struct DecodeLds {
   float b_scales[16 * KB];
   int b_target[16];  // pair of each route column, -1 = none
   int route_pairs[kMaxSlots];
-  int route_slots[MODE == 1 ? kMaxSlots : 1];
+  int route_slots[from_x(MODE) ? kMaxSlots : 1];
   int chunk_counts[kIdsPerThread * kGemmWaves];
 };
 
@@ -123,9 +136,11 @@ struct DecodeLds {
 // kEarly: the first weights are issued before the route scan (every
 // workgroup of an unsliced launch, slice 0 of a sliced one); otherwise only
 // after it, once the workgroup knows it has a route tile.
-template <int KB, int RT, int MODE, int TILES, int PASSES, bool kWholeFirst, bool kEarly>
-__device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<KB, MODE>& lds, int expert,
+template <int KB, int RT, int MODE, int TILES, int PASSES, bool kWholeFirst, bool kEarly, bool kPairGrid = false>
+__device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<KB, MODE>& lds, int unit,
                                                  int first_tile, int slice, int slices) {
+  static_assert(!kPairGrid || (MODE != 1 && kEarly), "the pair grid reads ids");
+  constexpr bool kFromX = from_x(MODE);
   const uint8_t* __restrict__ w = a.w;
   const float* __restrict__ ws = a.ws;
   const int n_rows = a.n_rows;
@@ -155,6 +170,35 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   const int group = lane >> 4;
   auto n0_of = [&](int tile) { return tile * kRowsPerGroup + wave * kRowsPerWave; };
 
+  // `unit`: the expert, or the pair whose expert this is (pair grid).  The
+  // expert's id is read as a vector load with the others (a scalar load would
+  // be a round trip of its own).
+  int expert = unit;
+  uint32_t pair_ids[kPairGridPairs / kWave];
+  uint64_t pair_hits[kPairGridPairs / kWave];
+  if constexpr (kPairGrid) {
+    const uint32_t words = static_cast<uint32_t>(capacity * top_k * a.id_words);
+    const BufferView id_view(a.ids, words * 4);
+    const uint32_t own = id_view.load4(static_cast<uint32_t>(unit * a.id_words) * 4);
+#pragma unroll
+    for (int c = 0; c < kPairGridPairs / kWave; ++c) {
+      const uint32_t word = static_cast<uint32_t>((c * kWave + lane) * a.id_words);
+      pair_ids[c] = id_view.load4(word < words ? word * 4 : kNoRow);
+    }
+    const int pairs = live_rows(a.row_count, capacity) * top_k;
+    expert = __builtin_amdgcn_readfirstlane(static_cast<int>(own));
+    if (unit >= pairs || expert < 0 || expert >= a.num_experts) return;  // uniform
+    bool earlier = false;
+#pragma unroll
+    for (int c = 0; c < kPairGridPairs / kWave; ++c) {
+      const int p = c * kWave + lane;
+      pair_hits[c] = __ballot(p < pairs && static_cast<int>(pair_ids[c]) == expert);
+      const int before = unit - c * kWave;  // pairs of this chunk before `unit`
+      const uint64_t mask = before <= 0 ? 0ull : (before >= kWave ? ~0ull : (1ull << before) - 1ull);
+      earlier |= (pair_hits[c] & mask) != 0ull;
+    }
+    if (earlier) return;  // uniform: an earlier pair's workgroup has this expert
+  }
   const uint8_t* wexp = w + static_cast<size_t>(expert) * n_rows * K;
   const float* wsexp = ws + static_cast<size_t>(expert) * (n_rows / kGroup) * KB;
   int32x8 a_frag[RT][KB];
@@ -328,19 +372,33 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
       }
     }
     routes = chunk_base;
+  } else if constexpr (kPairGrid) {
+    load_weights(first_tile, 0, kWholeFirst ? KB : kFirstHalf);
+    load_scales(first_tile, 0, kWholeFirst ? KB : kFirstHalf);
+    __builtin_amdgcn_sched_barrier(0);
+    routes = 0;
+#pragma unroll
+    for (int c = 0; c < kPairGridPairs / kWave; ++c) {
+      if (wave == 0 && ((pair_hits[c] >> lane) & 1ull)) {
+        const int r = routes + __popcll(pair_hits[c] & lanemask_lt());
+        route_pairs[r] = c * kWave + lane;
+        if constexpr (kFromX) route_slots[r] = (c * kWave + lane) / top_k;
+      }
+      routes += __popcll(pair_hits[c]);
+    }
   } else {
     // 1. The routed ids of every slot row (past the capacity: zeros, masked
     //    below), issued before any weight.
-    const uint32_t id_bytes = static_cast<uint32_t>(capacity * top_k) * 4;
+    const uint32_t id_bytes = static_cast<uint32_t>(capacity * top_k * a.id_words) * 4;
     const BufferView id_view(a.ids, id_bytes);
     uint32_t id[kIdsPerThread];
 #pragma unroll
     for (int j = 0; j < kIdsPerThread; ++j) {
-      const uint32_t p = static_cast<uint32_t>(j * kGemmThreads + threadIdx.x);
+      const uint32_t p = static_cast<uint32_t>(j * kGemmThreads + threadIdx.x) * a.id_words;
       id[j] = id_view.load4(p * 4 < id_bytes ? p * 4 : kNoRow);
     }
     const int rows = live_rows(a.row_count, capacity);
-    if (slice > 0 && first_route >= rows) return;  // at most one route per live row (uniform)
+    if (slice > 0 && first_route >= rows * a.row_routes) return;  // uniform
     // 2. The first half of the first weight tile streams meanwhile.
     if constexpr (kEarly) {
       load_weights(first_tile, 0, kWholeFirst ? KB : kFirstHalf);
@@ -369,8 +427,12 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
         base += w2 < wave ? c : 0;
         chunk_base += c;
       }
-      if ((hits[j] >> lane) & 1ull)
-        route_pairs[base + __popcll(hits[j] & lanemask_lt())] = j * kGemmThreads + threadIdx.x;
+      if ((hits[j] >> lane) & 1ull) {
+        const int r = base + __popcll(hits[j] & lanemask_lt());
+        const int pair = j * kGemmThreads + static_cast<int>(threadIdx.x);
+        route_pairs[r] = pair;
+        if constexpr (kFromX) route_slots[r] = pair / top_k;
+      }
     }
     routes = chunk_base;
   }
@@ -388,20 +450,23 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   float b_stage_scale = 0.0f;
   int stage_pair = -1;
   uint32_t stage_slot = 0;  // MODE 2 with row_slots: the slot of the route's row
-  // MODE 1: live (route column, 128-group) units packed densely as in MODE
+  // MODE 1 / 3: live (route column, 128-group) units packed densely as in MODE
   // 2; a unit's 16 threads hold 8 bf16 each (the front's quantisation
   // layout), so only live units are quantised.
-  constexpr int kStageUnits = MODE == 1 ? (KB < 8 ? KB : 8) : 1;  // unit rows staged at once
+  constexpr int kStageUnits = kFromX ? (KB < 8 ? KB : 8) : 1;  // unit rows staged at once
   uint4 x_stage[kStageUnits];
   // MODE 2: live (route column, K group) units packed densely: unit
   // u = 16 p + stage_col is column u / KB, group u % KB.
   uint4 g_stage[MODE == 2 ? KB : 1], u_stage[MODE == 2 ? KB : 1];
   int live_units = 0;
-  // MODE 1: unit rows [base, base + kStageUnits) of route tile stage_m0.
+  // MODE 1 / 3: unit rows [base, base + kStageUnits) of route tile stage_m0.
   int stage_m0 = 0;
   auto fetch_units = [&](int base) __attribute__((always_inline)) {
-    if constexpr (MODE == 1) {
-      const BufferView x_view(a.x, static_cast<uint32_t>(capacity * a.x_stride * 2));
+    if constexpr (kFromX) {
+      // MODE 1's last slot row may lie below the view's end by its stride's
+      // padding; MODE 3's view ends with the last row's data.
+      const BufferView x_view(a.x, static_cast<uint32_t>(
+                                       (MODE == 1 ? capacity * a.x_stride : (capacity - 1) * a.x_stride + K) * 2));
 #pragma unroll
       for (int i = 0; i < kStageUnits; ++i) {
         const int u = (base + i) * 16 + stage_col;
@@ -420,7 +485,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   // layout of quantize_row_part, so the tile holds the front's q bytes and
   // scales.
   auto quantize_units = [&](int base) __attribute__((always_inline)) {
-    if constexpr (MODE == 1) {
+    if constexpr (kFromX) {
 #pragma unroll
       for (int i = 0; i < kStageUnits; ++i) {
         if ((base + i) * 16 >= live_units) break;  // uniform
@@ -447,10 +512,10 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
       }
     }
   };
-  // MODE 1: the unit rows beyond the first kStageUnits (route tiles with
+  // MODE 1 / 3: the unit rows beyond the first kStageUnits (route tiles with
   // more than 128 / KB routes), staged and quantised after the rest.
   auto stage_rest = [&]() {
-    if constexpr (MODE == 1 && kStageUnits < KB) {
+    if constexpr (kFromX && kStageUnits < KB) {
       for (int base = kStageUnits; base < KB; base += kStageUnits) {
         if (base * 16 >= live_units) break;  // uniform
         fetch_units(base);
@@ -461,7 +526,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   auto fetch_tile = [&](int m0) {
     const int r = m0 + stage_col;
     stage_pair = r < routes ? route_pairs[r] : -1;
-    if constexpr (MODE == 1) {
+    if constexpr (kFromX) {
       live_units = min(16, routes - m0) * KB;
       stage_m0 = m0;
       fetch_units(0);
@@ -512,7 +577,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
           if (stage_part == 0) b_scales[col * KB + kb] = scale;
         }
       }
-    } else if constexpr (MODE == 1) {
+    } else if constexpr (kFromX) {
       quantize_units(0);
       stage_rest();
     } else {
@@ -653,7 +718,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   }
 }
 
-template <int KB, int RT, int MODE, int TILES, int PASSES = 1, bool kWholeFirst = false>
+template <int KB, int RT, int MODE, int TILES, int PASSES = 1, bool kWholeFirst = false, bool kPairGrid = false>
 __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2))) void decode_gemm_kernel(
     DecodeArgs a) {
   __shared__ DecodeLds<KB, MODE> lds;
@@ -666,6 +731,11 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2)
   // weight tile in its L2.
   const int slices = sliced_kernel(KB, MODE, TILES) && a.slices > 1 ? a.slices : 1;
   int unit = static_cast<int>(blockIdx.x), slice = 0;
+  if constexpr (kPairGrid) {
+    decode_gemm_body<KB, RT, MODE, TILES, PASSES, kWholeFirst, true, true>(a, lds, unit / groups,
+                                                                          (unit % groups) * TILES, 0, 1);
+    return;
+  }
   if (slices > 1) {
     const int units = a.num_experts * groups;
     const int stride = (units + 7) / 8 * 8;
@@ -746,9 +816,24 @@ int tiles_per_group(int num_experts, int tiles, int capacity, int top_k, int mod
   return 1;
 }
 
+// The pair grid: fewer pairs than experts, few enough for one workgroup's
+// ballots.
+bool pair_grid(int num_experts, int capacity, int top_k) {
+  return capacity * top_k <= kPairGridPairs && capacity * top_k < num_experts;
+}
+
 template <int KB, int MODE>
 void launch_decode(int num_experts, hipStream_t s, const DecodeArgs& a) {
   const int tiles = a.n_rows / tile_rows_for(KB);
+  if constexpr (MODE != 1) {
+    if (pair_grid(num_experts, a.capacity, a.top_k)) {
+      DecodeArgs args = a;
+      args.slices = 1;
+      hipLaunchKernelGGL((decode_gemm_kernel<KB, rt_for(KB), MODE, 1, 1, false, true>),
+                         dim3(a.capacity * a.top_k * tiles), dim3(kGemmThreads), 0, s, args);
+      return;
+    }
+  }
   const int t = tiles_per_group(num_experts, tiles, a.capacity, a.top_k, MODE);
   if constexpr (MODE != 2) {
     if (t == 6) {
@@ -973,6 +1058,8 @@ int check_expert_gemm(int32_t mode, const uint8_t* w, const float* ws, int32_t n
   args.exact_routes = exact_routes;
   args.num_experts = num_experts;
   args.ids = ids;
+  args.id_words = 1;
+  args.row_routes = 1;
   args.row_count = row_count;
   args.act = a;
   args.act_scales = a_scales;
@@ -987,6 +1074,9 @@ void launch_expert_gemm(const GemmLaunch& l, hipStream_t s) {
   if (l.mode == 0) {
     if (l.kb == 8) launch_decode<8, 0>(l.num_experts, s, l.args);
     else launch_decode<16, 0>(l.num_experts, s, l.args);
+  } else if (l.mode == 3) {
+    if (l.kb == 8) launch_decode<8, 3>(l.num_experts, s, l.args);
+    else launch_decode<16, 3>(l.num_experts, s, l.args);
   } else if (l.mode == 1) {
     if (l.kb == 8) launch_decode<8, 1>(l.num_experts, s, l.args);
     else launch_decode<16, 1>(l.num_experts, s, l.args);
@@ -1047,6 +1137,42 @@ int check_route_fc1(const uint8_t* w, const float* ws, int32_t num_experts, int3
   args.active_out = active;
   args.out_bf16 = gate_up;
   *launch = GemmLaunch{1, kb, num_experts, args};
+  return D3_OK;
+}
+
+// FC1 from given ids and bf16 rows (MODE 3): at most kPairGridPairs pairs, so
+// that an expert named by every pair still fits the route list.
+int check_ids_fc1(const uint8_t* w, const float* ws, int32_t num_experts, int32_t n, int32_t k,
+                  const uint16_t* x, int64_t x_stride, int32_t rows, const void* ids, int32_t ids_dtype,
+                  int32_t top_k, uint16_t* gate_up, GemmLaunch* launch) {
+  D3_REQUIRE(w && ws && x && ids && gate_up, "small_moe: null pointer");
+  D3_REQUIRE(ids_dtype == D3_DTYPE_I32 || ids_dtype == D3_DTYPE_I64, "small_moe: ids must be int32 or int64");
+  D3_REQUIRE(num_experts >= 1 && n > 0 && k > 0 && n % kGroup == 0 && k % 256 == 0,
+             "small_moe: N=%d must be a multiple of 128 and K=%d of 256", n, k);
+  D3_SUPPORTED(rows >= 1 && top_k >= 1 && top_k <= 8 && rows * top_k <= kPairGridPairs,
+               "small_moe: rows %d x top_k %d (<= 8) above %d routes", rows, top_k, kPairGridPairs);
+  D3_REQUIRE(x_stride >= k, "small_moe: row stride");
+  D3_SUPPORTED(aligned(x, 16) && x_stride % 8 == 0, "small_moe: x rows must be 16-byte aligned");
+  D3_SUPPORTED(static_cast<int64_t>(rows) * x_stride * 2 < (int64_t{1} << 31), "small_moe: rows above 2 GiB");
+  D3_REQUIRE(aligned(w, 16) && aligned(gate_up, 16), "small_moe: alignment");
+  const int kb = k / kGroup;
+  D3_SUPPORTED(kb == 8 || kb == 16, "small_moe: K=%d not in the compiled set", k);
+  D3_SUPPORTED(n % tile_rows_for(kb) == 0, "small_moe: N=%d must be a multiple of %d", n, tile_rows_for(kb));
+  DecodeArgs args{};
+  args.w = w;
+  args.ws = ws;
+  args.n_rows = n;
+  args.capacity = rows;
+  args.top_k = top_k;
+  args.exact_routes = kPairGridPairs;
+  args.num_experts = num_experts;
+  args.ids = static_cast<const int32_t*>(ids);
+  args.id_words = ids_dtype == D3_DTYPE_I64 ? 2 : 1;
+  args.row_routes = top_k;
+  args.x = x;
+  args.x_stride = x_stride;
+  args.out_bf16 = gate_up;
+  *launch = GemmLaunch{3, kb, num_experts, args};
   return D3_OK;
 }
 
@@ -1213,6 +1339,31 @@ extern "C" int d3_decode_expert_gemm(int32_t mode, const uint8_t* w, const float
   if (status != D3_OK) return status;
   launch_expert_gemm(launch, as_stream(stream));
   D3_LAUNCHED("decode_expert_gemm");
+}
+
+extern "C" int d3_small_moe(const uint8_t* w13, const float* s13, const uint8_t* w2, const float* s2,
+                            int32_t num_experts, int32_t hidden, int32_t intermediate, const uint16_t* x,
+                            int64_t x_stride, int32_t rows, const void* ids, int32_t ids_dtype,
+                            const void* weights, int32_t weights_dtype, int32_t top_k, uint16_t* gate_up,
+                            float* down, uint16_t* out, void* stream) {
+  D3_REQUIRE(hidden > 0 && intermediate > 0, "small_moe: hidden %d, intermediate %d", hidden, intermediate);
+  D3_REQUIRE(weights && down && out, "small_moe: null pointer");
+  D3_REQUIRE(weights_dtype == D3_DTYPE_BF16 || weights_dtype == D3_DTYPE_F32,
+             "small_moe: weights must be bf16 or f32");
+  D3_REQUIRE(aligned(out, 8), "small_moe: output alignment");
+  GemmLaunch fc1{}, fc2{};
+  int status = check_ids_fc1(w13, s13, num_experts, 2 * intermediate, hidden, x, x_stride, rows, ids, ids_dtype,
+                             top_k, gate_up, &fc1);
+  if (status != D3_OK) return status;
+  status = check_expert_gemm(2, w2, s2, num_experts, hidden, intermediate, fc1.args.ids, nullptr, nullptr, rows,
+                             top_k, gate_up, nullptr, kPairGridPairs, nullptr, down, &fc2);
+  if (status != D3_OK) return status;
+  fc2.args.id_words = fc1.args.id_words;
+  fc2.args.row_routes = top_k;
+  hipStream_t s = as_stream(stream);
+  launch_expert_gemm(fc1, s);
+  launch_expert_gemm(fc2, s);
+  return d3_weighted_combine(down, weights, weights_dtype, rows, top_k, hidden, nullptr, nullptr, out, stream);
 }
 
 extern "C" int d3_decode_route_fc1(const uint8_t* w, const float* ws, int32_t num_experts,

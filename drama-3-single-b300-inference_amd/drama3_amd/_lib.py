@@ -77,6 +77,9 @@ SIGNATURES = {
         _i32, [_p, _p, _i32, _i32, _i32, _i32, _p, _p, _i32, _p, _p, _i32, _i32, _i32, _p, _p]),
     "d3_decode_expert_gemm": (
         _i32, [_i32, _p, _p, _i32, _i32, _i32, _p, _p, _p, _i32, _i32, _p, _p, _i32, _p, _p, _p]),
+    "d3_small_moe": (
+        _i32, [_p, _p, _p, _p, _i32, _i32, _i32, _p, _i64, _i32, _p, _i32, _p, _i32, _i32, _p, _p,
+               _p, _p]),
     "d3_decode_route_fc1": (
         _i32, [_p, _p, _i32, _i32, _i32, _p, _i32, _p, _i64, _p, _i32, _i64, _i32, _i32, _p, _p,
                _p, _p, _p]),

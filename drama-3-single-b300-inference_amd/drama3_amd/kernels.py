@@ -14,10 +14,14 @@ import torch
 
 from . import _lib
 from ._lib import call, ptr
-from .pipeline import (WIDE_SORT_PAIRS, MoEWorkspace, Shape, by_pair_suited, dtype_code,
-                       grouped_supported, require_cuda)
+from .pipeline import (SORTLESS_PAIRS, WIDE_SORT_PAIRS, MoEWorkspace, Shape, by_pair_suited,
+                       dtype_code, fragment_weights, grouped_supported, require_cuda,
+                       sortless_suited)
 
 TOP_K = 8
+# Most rows of routed_moe without a route sort (no expert has more routes than
+# rows, so every expert stays on the exact path).
+SORTLESS_ROWS = 64
 
 # Workspaces of the eager entry points, reused across calls with the same
 # shape, options, device and current stream (calls on one stream run in
@@ -116,6 +120,9 @@ def _routed(x, topk_ids, topk_weights, experts, block_m: int = 16):
     ids, weights = topk_ids.contiguous(), topk_weights.contiguous()
     if x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
+    if (rows * top_k <= SORTLESS_PAIRS and sortless_suited(rows, e, h, i, top_k)
+            and fragment_weights(experts)):
+        return ws.small_forward(x, ids, weights, experts, out)
     return ws.experts_forward(x, ids, weights, experts, out=out)
 
 
@@ -307,6 +314,10 @@ def routed_moe(x, router, experts, decode=True, *, row_slots=None, padding_start
                                          padding_start=padding_start)
     if x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
+    if (rows <= SORTLESS_ROWS and sortless_suited(rows, e, h, i, TOP_K)
+            and fragment_weights(experts)):
+        ws = _workspace(Shape(rows, e, h, i, TOP_K), x.device, sortless=True)
+        return ws.forward(x, logits, experts, out=out)
     by_pair = by_pair_suited(rows, e, TOP_K) and grouped_supported(h, i)
     ws = _workspace(Shape(rows, e, h, i, TOP_K), x.device,
                     item_rows=128 if rows > 128 else None, by_pair=by_pair)

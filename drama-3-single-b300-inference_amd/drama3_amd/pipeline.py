@@ -101,6 +101,30 @@ def default_item_rows(rows: int, tile: int = SORT_TILE, num_experts: int | None 
     return max(tile, -(-rows // tile) * tile)
 
 
+SORTLESS_PAIRS = 256  # most (row, rank) pairs of the expert GEMMs' pair grid
+
+
+def sortless_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
+                    top_k: int = 8) -> bool:
+    """Whether the expert GEMMs without a route sort (d3_decode_expert_gemm,
+    fragment-major weights) suit a batch: compiled shapes, and either at least
+    one route per expert on average (each expert's workgroups look for its
+    routes) or few enough pairs for the pair grid (a workgroup per pair)."""
+    lib = _lib.load()
+    shapes = (hidden // 128 in (8, 16) and intermediate // 128 in (2, 4, 6, 8)
+              and hidden % 128 == 0 and intermediate % 128 == 0
+              and hidden % lib.d3_expert_tile_rows(intermediate) == 0)
+    pairs = rows * top_k
+    return (shapes and rows <= 256 and top_k <= 8
+            and (pairs >= num_experts or pairs <= SORTLESS_PAIRS))
+
+
+def fragment_weights(experts) -> bool:
+    """Whether both weight tensors have fragment-major copies."""
+    return (fc1_operands(experts)[2] == LAYOUT_FRAGMENT
+            and fc2_operands(experts)[2] == LAYOUT_FRAGMENT)
+
+
 @dataclass
 class Shape:
     rows: int
@@ -398,6 +422,18 @@ class MoEWorkspace:
             self._fc2_stage(experts, stream)
         return self.combine(weights, row_count, shared, out, stream)
 
+    def small_forward(self, x, ids, weights, experts, out, stream=None) -> torch.Tensor:
+        """Given routes of a handful of rows, fragment-major weights: FC1 that
+        quantises its rows itself, FC2 and combine, without a route sort."""
+        s, stream = self.shape, self._stream(stream)
+        w13, s13, _ = fc1_operands(experts)
+        w2, s2, _ = fc2_operands(experts)
+        call("d3_small_moe", ptr(w13), ptr(s13), ptr(w2), ptr(s2), s.num_experts, s.hidden,
+             s.intermediate, ptr(x), x.stride(0), s.rows, ptr(ids), dtype_code(ids.dtype),
+             ptr(weights), dtype_code(weights.dtype), s.top_k, ptr(self.gate_up), ptr(self.down),
+             ptr(out), stream)
+        return out
+
     def _fc2_stage(self, experts, stream) -> None:
         if self.swiglu_in_fc2:
             self.fc2_swiglu(experts, stream)
@@ -664,21 +700,19 @@ class DecodeStep:
         # FP8-only tiled grouped GEMMs of prefill-sized batches).
         self.workspace = MoEWorkspace(Shape(slots, num_experts, hidden, intermediate, top_k), dev,
                                       item_rows=item_rows, grouped=False)
-        # Sortless expert GEMMs (default when the slots' routes could reach
-        # every expert: at least one route per expert at full occupancy, and
-        # the shapes are in the compiled set) on fragment-major weights.
-        # Measured at 64 slots: E128 (8 routes per expert) and the reference
-        # model's E256 / I512 (2 per expert: 127 us against 134 us for the
-        # sorted chain).
-        lib = _lib.load()
-        decode_shapes = (hidden // 128 in (8, 16) and intermediate // 128 in (2, 4, 6, 8)
-                         and hidden % 128 == 0 and intermediate % 128 == 0
-                         and hidden % lib.d3_expert_tile_rows(intermediate) == 0)
-        dense = slots * top_k >= num_experts
+        # Sortless expert GEMMs on fragment-major weights whenever the shapes
+        # and the batch suit them (sortless_suited).  Measured at 64 slots:
+        # E128 (8 routes per expert) and the reference model's E256 / I512 (2
+        # per expert: 127 us against 134 us for the sorted chain).
+        suited = sortless_suited(slots, num_experts, hidden, intermediate, top_k)
         if sortless is None:
-            sortless = decode_shapes and dense and slots <= 256 and top_k <= 8
+            sortless = suited
         self.sortless = bool(sortless)
-        self.frontless = self.sortless if frontless is None else bool(frontless)
+        # The FC1 from the slots has a workgroup per expert, which pays when the
+        # slots' routes reach most of them.
+        if frontless is None:
+            frontless = self.sortless and slots * top_k >= num_experts
+        self.frontless = bool(frontless)
         if self.frontless and not self.sortless:
             raise ValueError("frontless runs the sortless chain (sortless=True)")
 
@@ -716,8 +750,7 @@ class DecodeStep:
 
     @staticmethod
     def uses_sortless_layout(experts) -> bool:
-        return (fc1_operands(experts)[2] == LAYOUT_FRAGMENT
-                and fc2_operands(experts)[2] == LAYOUT_FRAGMENT)
+        return fragment_weights(experts)
 
     def uses_sortless(self, experts) -> bool:
         return self.sortless and self.uses_sortless_layout(experts)

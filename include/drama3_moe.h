@@ -451,6 +451,27 @@ int d3_decode_expert_gemm(int32_t mode, const uint8_t *w, const float *ws, int32
                           uint16_t *out_bf16, float *out_f32, void *stream);
 
 /*
+ * A4, A8-A11  The routed experts of a handful of rows with given routes
+ * (three launches, no route sort): small_batch_moe
+ * (src/drama3/kernels.py:325-357).  FC1 quantises the bf16 rows of its
+ * routes while staging them and finds them in the ids (a workgroup per
+ * (pair, weight tile) where there are fewer pairs than experts, else per
+ * (expert, weight tile)), FC2 takes the SwiGLU requant in its prologue, then
+ * d3_weighted_combine.  Every expert contracts on the exact path.
+ *   w13 / w2 fragment-major; x bf16 [rows, x_stride] (16-byte aligned rows);
+ *   ids int32 or int64 [rows, top_k] (an expert may repeat in a row; pairs
+ *   with an id outside [0, E) are skipped), weights bf16 or f32 [rows, top_k];
+ *   gate_up bf16 [rows * top_k, 2I], down f32 [rows * top_k, H]: scratch;
+ *   out bf16 [rows, H].  rows * top_k <= 256, top_k <= 8, H in {1024, 2048},
+ *   I in {256, 512, 768, 1024}.
+ */
+int d3_small_moe(const uint8_t *w13, const float *s13, const uint8_t *w2, const float *s2,
+                 int32_t num_experts, int32_t hidden, int32_t intermediate, const uint16_t *x,
+                 int64_t x_stride, int32_t rows, const void *ids, int32_t ids_dtype,
+                 const void *weights, int32_t weights_dtype, int32_t top_k, uint16_t *gate_up,
+                 float *down, uint16_t *out, void *stream);
+
+/*
  * A1-A3, A5, A8  Decode FC1 straight from the slots (no front launch).
  * Replaces, for the decode step, the slot filter (src/drama3/engine.py:637-647),
  * route_kernel's top-k (src/drama3/kernels.py:360-383), the per-128

@@ -318,3 +318,61 @@ def test_standalone_entries_match_the_step(device):
     ws.decode_fc2(experts, parts.count)
     torch.cuda.synchronize()
     assert torch.equal(ws.down[:8 * n].view(torch.int32), whole.workspace.down[by_slot].view(torch.int32))
+
+
+@pytest.mark.parametrize("ids_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("rows,experts,repeats", [(1, 256, False), (5, 256, True), (31, 256, False),
+                                                  (32, 256, False), (32, 128, False), (9, 16, False),
+                                                  (32, 16, True), (32, 4, True)])
+def test_small_moe_matches_sorted_chain(device, rows, experts, repeats, ids_dtype):
+    """The sortless chain from given ids (pair grid below one route per
+    expert, expert grid from there) against the sorted chain, bit for bit:
+    strided x rows, both id types, rows that repeat an expert (up to every
+    pair on one expert)."""
+    from drama3_amd.expert_weights import prepare_experts
+    from drama3_amd.pipeline import MoEWorkspace, Shape
+    from drama3_amd.workloads import make_experts
+
+    gen = torch.Generator("cpu").manual_seed(31 * rows + experts)
+    h, i, top_k = 1024, 256, 8
+    weights = torch.rand((rows, top_k), generator=gen).to(device)
+    if repeats:
+        ids = torch.randint(0, experts, (rows, top_k), generator=gen)
+        ids[rows // 2:] = experts - 1
+    else:
+        ids = torch.stack([torch.randperm(experts, generator=gen)[:top_k] for _ in range(rows)])
+    ids = ids.to(device=device, dtype=ids_dtype)
+    x = torch.randn((rows, h + 8), generator=gen).to(torch.bfloat16).to(device)[:, :h]
+    packed = prepare_experts(make_experts(gen, experts, h, i).to(device))
+    shape = Shape(rows, experts, h, i, top_k)
+    small, chain = (MoEWorkspace(shape, device, item_rows=16) for _ in range(2))
+    got, expected = (torch.empty((rows, h), dtype=torch.bfloat16, device=device) for _ in range(2))
+    small.small_forward(x, ids, weights, packed, got)
+    chain.experts_forward(x, ids, weights, packed, out=expected)
+    torch.cuda.synchronize()
+    assert torch.equal(small.down.view(torch.int32), chain.down.view(torch.int32))
+    assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
+
+
+@pytest.mark.parametrize("slots,live", [(1, 1), (16, 11), (31, 31), (32, 20)])
+def test_few_slots_match_sorted_chain(device, slots, live):
+    """Fewer routes than experts: DecodeStep runs the pair grid after the
+    front; every byte as the sorted chain's."""
+    from drama3_amd.expert_weights import prepare_experts
+    from drama3_amd.pipeline import DecodeStep
+    from drama3_amd.workloads import make_experts
+
+    gen = torch.Generator("cpu").manual_seed(slots)
+    e, h, i = 272, 1024, 512
+    packed = prepare_experts(make_experts(gen, e, h, i).to(device))
+    few = DecodeStep(slots, e, h, i, device=device)
+    assert few.uses_sortless(packed) and not few.frontless
+    chain = DecodeStep(slots, e, h, i, device=device, sortless=False)
+    occupancy = torch.zeros(slots, dtype=torch.uint8)
+    occupancy[torch.randperm(slots, generator=gen)[:live]] = 1
+    xs = torch.randn((slots, h), generator=gen).to(torch.bfloat16).to(device)
+    ls = torch.randn((slots, e), generator=gen).to(torch.bfloat16).to(device)
+    for step in (few, chain):
+        step(occupancy.to(device), xs, ls, packed)
+    torch.cuda.synchronize()
+    assert compare(few, chain) == live
