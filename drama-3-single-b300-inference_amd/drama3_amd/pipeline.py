@@ -109,13 +109,21 @@ def sortless_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
     """Whether the expert GEMMs without a route sort (d3_decode_expert_gemm,
     fragment-major weights) suit a batch: compiled shapes, and either at least
     one route per expert on average (each expert's workgroups look for its
-    routes) or few enough pairs for the pair grid (a workgroup per pair)."""
+    routes) or few enough pairs for the pair grid (a workgroup per pair).
+
+    Many experts with eight or more routes each, from more than 64 rows, are
+    the sorted chain's: the sortless GEMMs then walk their weight tiles again
+    for experts beyond 16 routes (step, sortless -> sorted: E128 128 rows 144
+    -> 126 us, 256 rows 221 -> 140 us; E256 256 rows 160 us either way; E128
+    100 rows, 6 per expert, 112 against 122 us).  With few experts their
+    route slices run side by side instead (E16: 26 against 42 us)."""
     lib = _lib.load()
     shapes = (hidden // 128 in (8, 16) and intermediate // 128 in (2, 4, 6, 8)
               and hidden % 128 == 0 and intermediate % 128 == 0
               and hidden % lib.d3_expert_tile_rows(intermediate) == 0)
     pairs = rows * top_k
-    return (shapes and rows <= 256 and top_k <= 8
+    busy = rows > 64 and num_experts >= 64 and pairs >= 8 * num_experts
+    return (shapes and rows <= 256 and top_k <= 8 and not busy
             and (pairs >= num_experts or pairs <= SORTLESS_PAIRS))
 
 
