@@ -44,8 +44,8 @@ __global__ __launch_bounds__(kSortThreads) void sort_routes_kernel(
 //      and per expert.  Every workgroup reads all chunk histograms (thread e
 //      sums its expert's column, and the part of it above its own chunk), so
 //      each holds the padded expert scan and its chunk's offsets itself:
-//      sorted_ids[start[e] + chunk offset + rank] = p.  The last workgroup
-//      also writes the sentinel padding, expert ids, work items and totals.
+//      sorted_ids[start[e] + chunk offset + rank] = p, and writes its share
+//      of the sentinel padding, expert ids, work items and totals.
 //      (A single workgroup scanning the histograms between two launches, as
 //      before, took 8 us of a 13 us pair at config 4.)
 // Scratch: chunk histograms [chunks][E] and ranks [pairs] (int32).
@@ -185,9 +185,8 @@ __global__ __launch_bounds__(kPlaceThreads) void wide_place_kernel(
       if (out.inverse != nullptr) out.inverse[p] = position;
     }
   }
-  if (mine == static_cast<int>(gridDim.x) - 1)
-    write_sort_tail<kPlaceThreads, false>(counts, starts, first_item, num_experts, tile, item_rows, total,
-                                          total_items, pairs, out);
+  write_sort_tail<kPlaceThreads, false>(counts, starts, first_item, num_experts, tile, item_rows, total, total_items,
+                                        pairs, out, mine, static_cast<int>(gridDim.x));
 }
 
 }  // namespace
