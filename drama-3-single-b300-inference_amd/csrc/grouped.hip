@@ -2,13 +2,18 @@
 // mixed batches): work items of up to 128 sorted routes against 256 weight
 // rows, the contraction streamed in 128-byte K blocks.
 //
+// Two kernels: grouped_items_kernel over the route sort's work items (FC1 and
+// FC2), and grouped_by_pair_kernel (FC1 of small batches, which finds its
+// routes itself and writes them as items for FC2).
+//
 // Design (gfx950, wave64, MFMA 16x16x128 OCP-FP8, 4 waves per workgroup,
 // two workgroups per CU):
 //   * A workgroup owns (work item, weight row tile).  Each wave owns four
 //     16-row weight tiles (FC1: two gate tiles and the matching two up
-//     tiles) and all eight 16-route tiles of the item: 32 MFMAs per K block,
-//     128 fp32 accumulators per lane; each B fragment read from LDS feeds
-//     four MFMAs.
+//     tiles) and every 16-route tile of the item, in the smallest of four
+//     bodies that holds it (2, 4, 6 or 8 route tiles): at 8, 32 MFMAs per K
+//     block and 128 fp32 accumulators per lane; each B fragment read from
+//     LDS feeds four MFMAs.
 //   * Weights go straight from memory into MFMA fragments one K block ahead
 //     of the MFMAs (fragment-major layout: two 1 KiB contiguous loads per
 //     tile and K block; checkpoint layout: 16 rows x 64 bytes per load).
@@ -17,11 +22,13 @@
 //     two-slot LDS ring (128 routes x 144-byte rows; the 16-byte pad keeps
 //     the 16 rows of each ds_read_b128 on distinct banks); their loads are
 //     issued before the weights', so waiting for them never waits for the
-//     weights.  The next block's loads are issued in units spread over the
-//     current block's route tiles (one activation copy or one weight tile
-//     per route tile): issued in one block at its top they held the wave's
-//     MFMAs back while the memory pipeline drained (3 % slower per GEMM).
-//     One barrier per K block.
+//     weights.  In the contraction-sized bodies (6 and 8 route tiles) the
+//     next block's loads are issued in units spread over the current block's
+//     route tiles (one activation copy or one weight tile per route tile):
+//     issued in one block at its top they held the wave's MFMAs back while
+//     the memory pipeline drained (3 % slower per GEMM).  The smaller bodies
+//     keep two or three K blocks in flight in the registers they save.  One
+//     barrier per K block.
 //   * Measured per workgroup (per-workgroup timestamps, config-4 FC1): the
 //     prologue (item, route ids, scales, first blocks) and the epilogue
 //     cost a third of a workgroup's time; two resident workgroups per CU
@@ -61,16 +68,16 @@ constexpr int kGgStride = kGroup + 16;             // LDS bytes per staged route
 constexpr int kGgRowF = kGgRows + 4;               // floats per route row of FC2's epilogue buffers
 static_assert(2 * 16 * kGgRowF * 4 <= 2 * kGgRoutes * kGgStride, "two epilogue buffers fit the staging ring");
 constexpr int kGgXcds = 8;
-// Launches whose experts average at most this many routes at capacity run
-// the sparse kernel, if they fill a round of resident workgroups (two per
-// CU): below one round the launch is a single prologue and K loop, which the
-// 128-route kernel runs 0.5 us faster (E16 H1024 I256, 140 rows: FC1 15.7
-// against 16.1 us).  Kernel trace, FC1 / FC2 us, 128-route kernel -> sparse:
-// E256 I512 3,000 rows (94 routes per expert) 119.5 / 95.7 -> 114.5 / 88.0,
-// 3,300 rows (103) 123.3 / 98.5 -> 120.2 / 93.6, 3,600 rows (113) 137.3 /
-// 100.9 -> 138.5 / 98.7; E128 I768 1,500 rows (94) 96.6 / 64.3 -> 92.0 / 62.0,
-// 1,700 rows (106) 97.5 / 71.1 -> 98.1 / 71.5, 1,900 rows (119) 99.7 / 71.6
-// -> 110.6 / 77.4.
+// Launches whose experts average at most this many routes at capacity read
+// their weights non-temporally and with more blocks in flight
+// (grouped_items_kernel, kSparse), if they fill a round of resident workgroups
+// (two per CU): below one round the launch is one prologue and K loop, 0.5 us
+// faster the other way (E16 H1024 I256, 140 rows).  Kernel trace, FC1 / FC2
+// us, dense -> sparse: E256 I512 3,000 rows (94 routes per expert) 119.5 / 95.7
+// -> 114.5 / 88.0, 3,300 rows (103) 123.3 / 98.5 -> 120.2 / 93.6, 3,600 rows
+// (113) 137.3 / 100.9 -> 138.5 / 98.7; E128 I768 1,500 rows (94) 96.6 / 64.3 ->
+// 92.0 / 62.0, 1,700 rows (106) 97.5 / 71.1 -> 98.1 / 71.5, 1,900 rows (119)
+// 99.7 / 71.6 -> 110.6 / 77.4.
 constexpr int kSparseRoutes = 104;
 constexpr int kResidentGroups = 512;
 constexpr int kStreamOutRoutes = 16384;  // FC2 launches up to this many item routes stream their rows
@@ -170,40 +177,36 @@ __device__ __forceinline__ void store_fc1(const floatx4 (&acc)[kGgWaveTiles][kRT
   }
 }
 
-// kByPair (FC1 of small batches): no sorted route list.  A work item is
-// part j (routes [64 j, 64 j + 64) in pair order) of an expert; the
-// workgroup finds those routes itself in `sorted_ids`, which
-// then holds the routed expert of every (row, rank) pair, the live row
-// count being *num_items.  What they found is written out as a sorted
+// FC1 of small batches without a sorted route list.  A work item is part j
+// (routes [64 j, 64 j + 64) in pair order) of an expert; the workgroup finds
+// those routes itself in `ids`, the routed expert of every (row, rank) pair
+// of the *row_count live rows.  What they found is written out as a sorted
 // route list of 128-route items, two parts each - item i = (expert, 128 i,
 // routes), its pairs at list_ids[128 i ..] in ascending order - and FC1
 // writes act rows at those positions, so the sorted FC2 launch reads them
 // as it reads a route sort's.
-// kStreamOut (FC2): the fp32 rows go out with non-temporal stores.
-template <int KB, int MODE, bool kPacked, bool kByPair, bool kStreamOut = false>
-__global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2))) void grouped_gemm_kernel(
+template <int KB, bool kPacked>
+__global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2))) void grouped_by_pair_kernel(
     const uint8_t* __restrict__ w, const float* __restrict__ ws, int n_rows, int out_cols,
     const uint8_t* __restrict__ act, uint32_t act_bytes, const float* __restrict__ act_scales,
-    const int32_t* __restrict__ sorted_ids, int top_k, const int4* __restrict__ items,
-    const int32_t* __restrict__ num_items, int max_items, SharedItems shared, int n_tiles, int chunk,
-    int parts, int capacity, int32_t* __restrict__ list_ids, int4* __restrict__ list_items,
-    int32_t* __restrict__ list_count, uint8_t* __restrict__ out_codes, float* __restrict__ out_scales,
-    float* __restrict__ out_f32) {
-  static_assert(!kByPair || MODE == 0, "the route lists come from FC1");
+    const int32_t* __restrict__ route_ids, int top_k, const int32_t* __restrict__ row_count, int max_items,
+    int n_tiles, int chunk, int parts, int capacity, int32_t* __restrict__ list_ids,
+    int4* __restrict__ list_items, int32_t* __restrict__ list_count, uint8_t* __restrict__ out_codes,
+    float* __restrict__ out_scales) {
   constexpr int K = KB * kGroup;
-  // Routes per work item: by-pair launches take 64 (twice the workgroups,
-  // each with half the epilogue, for batches that leave most CUs idle).
-  constexpr int kR = kByPair ? kGgPairRoutes : kGgRoutes;
+  // 64 routes per work item (twice the workgroups of 128, each with half the
+  // epilogue, for batches that leave most CUs idle).
+  constexpr int kR = kGgPairRoutes;
   constexpr int kRT = kR / 16;                              // 16-route tiles per wave
   constexpr int kStage = kR * kGgStride;
   constexpr int kStaged = kR * kGroup / (16 * kGgThreads);  // 16-byte copies per thread and K block
   __shared__ __attribute__((aligned(16))) uint8_t stage[2][kStage];
   __shared__ float a_scale[KB][kR];
-  __shared__ int target[kR];  // FC1: sorted position, FC2: pair; -1 = no route
-  __shared__ float amax_part[MODE == 0 ? kGgWaves : 1][kR];
-  __shared__ int route_pair[kByPair ? kR : 1];
-  __shared__ uint64_t chunk_masks[kByPair ? kGgMaxPairChunks * kGgWaves : 1];
-  __shared__ int chunk_base[kByPair ? kGgMaxPairChunks * kGgWaves + 1 : 1];
+  __shared__ int target[kR];  // list position, -1 = no route
+  __shared__ float amax_part[kGgWaves][kR];
+  __shared__ int route_pair[kR];
+  __shared__ uint64_t chunk_masks[kGgMaxPairChunks * kGgWaves];
+  __shared__ int chunk_base[kGgMaxPairChunks * kGgWaves + 1];
 
   // XCD-aware order: workgroup b runs on XCD b % 8; logical index L gives
   // each XCD runs of `chunk` = 2 n_tiles consecutive workgroups: the tiles
@@ -215,34 +218,15 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
   const int within = logical % chunk;
   const int item_index = (logical / chunk) * 2 + (within & 1);
   const int tile = within >> 1;
-  const bool dense = item_index >= max_items;  // a shared-expert item (uniform)
-  int expert = 0, first = 0, routes = 0;
-  int pj = 0, slot = 0;  // by-pair: the expert's part, and its expert-major index
-  if constexpr (kByPair) {
-    if (item_index >= max_items) return;
-    // Part-pair-major order (parts 2 p and 2 p + 1 of every expert, then
-    // the next p): the launch's first workgroups take the parts that hold
-    // routes, so they start on CUs of their own.
-    const int experts_n = max_items / parts;
-    const int pp = item_index / (2 * experts_n), rem = item_index - pp * 2 * experts_n;
-    expert = rem >> 1;
-    pj = 2 * pp + (rem & 1);
-    slot = expert * parts + pj;
-  } else if (!dense) {
-    // The item is read together with the item count (item_index <
-    // max_items: in bounds) and both decide the one early exit, so both
-    // loads are in flight at once: one memory round trip, not two.
-    const int4 item = items[item_index];
-    const int count = *num_items;
-    expert = item.x;
-    first = item.y;
-    routes = item_index < count ? min(item.z, kR) : 0;
-    if (routes <= 0) return;  // a padding item (uniform)
-  } else {
-    first = (item_index - max_items) * kR;
-    if (first >= shared.rows) return;
-    routes = min(kR, shared.rows - first);
-  }
+  if (item_index >= max_items) return;
+  // Part-pair-major order (parts 2 p and 2 p + 1 of every expert, then the
+  // next p): the launch's first workgroups take the parts that hold routes,
+  // so they start on CUs of their own.
+  const int experts_n = max_items / parts;
+  const int pp = item_index / (2 * experts_n), rem = item_index - pp * 2 * experts_n;
+  const int expert = rem >> 1;
+  const int pj = 2 * pp + (rem & 1);      // the expert's part
+  const int slot = expert * parts + pj;  // and its expert-major index
 
   const int tid = threadIdx.x;
   const int lane = lane_id();
@@ -251,15 +235,12 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
   const int group = lane >> 4;
 
   // Weight rows of this wave's tile t (16 rows each).
-  const int n0 = tile * (MODE == 0 ? kGroup : kGgRows);
-  auto tile_row = [&](int t) {
-    if constexpr (MODE == 0)  // t = 0, 1: gate rows; t = 2, 3: the matching up rows
-      return (t < 2 ? 0 : out_cols) + n0 + 32 * wave + 16 * (t & 1);
-    else
-      return n0 + 64 * wave + 16 * t;
+  const int n0 = tile * kGroup;
+  auto tile_row = [&](int t) {  // t = 0, 1: gate rows; t = 2, 3: the matching up rows
+    return (t < 2 ? 0 : out_cols) + n0 + 32 * wave + 16 * (t & 1);
   };
-  const uint8_t* wexp = dense ? shared.w : w + static_cast<size_t>(expert) * n_rows * K;
-  const float* wsexp = dense ? shared.ws : ws + static_cast<size_t>(expert) * (n_rows / kGroup) * KB;
+  const uint8_t* wexp = w + static_cast<size_t>(expert) * n_rows * K;
+  const float* wsexp = ws + static_cast<size_t>(expert) * (n_rows / kGroup) * KB;
 
   // Weight fragments through a buffer view of the expert: the lane offset
   // is one VGPR, the tile / K block offset a wave-uniform scalar.  Loads are
@@ -288,17 +269,16 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
       wf[kb & 1][t] = v;
     }
   };
-  if constexpr (!kByPair) load_weights(0);  // depends on the item only
-
-  if constexpr (kByPair) {
+  int routes;
+  {
     // The expert's routes in pair order: pair p = 256 j + thread.  Each
     // wave's ballot of chunk j goes to LDS; one wave turns their counts into
     // exclusive bases (in pair order: chunk, then wave); each thread then
     // ranks only its own matches (a few of its 32 chunks).
     const int part_first = pj * kR;
-    const int live_rows = min(*num_items, capacity);
+    const int live_rows = min(*row_count, capacity);
     const int pairs = live_rows * top_k;
-    const BufferView id_view(sorted_ids, static_cast<uint32_t>(capacity * top_k) * 4);
+    const BufferView id_view(route_ids, static_cast<uint32_t>(capacity * top_k) * 4);
     const int my_wave = static_cast<int>(threadIdx.x) / kWave;
     uint32_t mine = 0;  // bit j: this thread's pair of chunk j routes to the expert
     {
@@ -361,27 +341,18 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
   }
 
   // Route rows of the item, loaded branch-free (a dead route reads the
-  // item's first id and is masked afterwards): one round trip.  Shared-expert
-  // items map row r of the item to token first + r.
-  auto route_row = [&](int r, int id) {
-    if (dense) return MODE == 0 ? first + r : shared.pos + first + r;
-    return MODE == 0 ? id / top_k : first + r;
-  };
+  // item's first id and is masked afterwards): one round trip.
   const int part = tid & 7;
   const int r0 = tid >> 3;
   int ids[kStaged];
 #pragma unroll
   for (int i = 0; i < kStaged; ++i) {
     const int r = r0 + (kGgThreads / 8) * i;
-    if constexpr (kByPair)
-      ids[i] = route_pair[r < routes ? r : 0];
-    else
-      ids[i] = dense ? 0 : sorted_ids[first + (r < routes ? r : 0)];
+    ids[i] = route_pair[r < routes ? r : 0];
   }
   const int rs = tid % kR;       // route of this thread's scales / target
   const int k0 = tid / kR;       // first K block of its scales
-  const int id_s = kByPair ? route_pair[rs < routes ? rs : 0]
-                           : (dense ? 0 : sorted_ids[first + (rs < routes ? rs : 0)]);
+  const int id_s = route_pair[rs < routes ? rs : 0];
 
   // Staging: thread t copies 16 bytes (chunk t % 8 of the K block) of routes
   // t / 8 + 32 i.  Dead routes read past the buffer (zeros).
@@ -390,7 +361,7 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
   for (int i = 0; i < kStaged; ++i) {
     const int r = r0 + (kGgThreads / 8) * i;
-    src[i] = r < routes ? static_cast<uint32_t>(route_row(r, ids[i])) * K + part * 16 : kNoRow;
+    src[i] = r < routes ? static_cast<uint32_t>(ids[i] / top_k) * K + part * 16 : kNoRow;
   }
   int4 staged[kStaged];
   auto stage_load = [&](int kb) {
@@ -409,19 +380,17 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
   {
     constexpr int kSplit = kGgThreads / kR;  // threads per route row of scales
     const bool live = rs < routes;
-    const float* srow = act_scales + static_cast<size_t>(route_row(rs, id_s)) * KB;
+    const float* srow = act_scales + static_cast<size_t>(id_s / top_k) * KB;
     float sc[(KB + kSplit - 1) / kSplit];
 #pragma unroll
     for (int q = 0; q * kSplit + k0 < KB; ++q) sc[q] = srow[q * kSplit + k0];
 #pragma unroll
     for (int q = 0; q * kSplit + k0 < KB; ++q) a_scale[q * kSplit + k0][rs] = live ? sc[q] : 0.0f;
-    int t = MODE == 1 ? id_s : (kByPair ? slot * kR : first) + rs;
-    if (dense) t = (MODE == 0 ? shared.pos : shared.pair) + first + rs;
+    const int t = slot * kR + rs;
     if (k0 == 0) target[rs] = live ? t : -1;
   }
-  // Block scales of the wave's tiles for every K block (wave-uniform): FC1
-  // tiles 0-1 (gate) share one 128-row block and tiles 2-3 (up) another; a
-  // wave's four FC2 tiles lie in one block.
+  // Block scales of the wave's tiles for every K block (wave-uniform): tiles
+  // 0-1 (gate) share one 128-row block and tiles 2-3 (up) another.
   float w_rows[2][KB];
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
@@ -508,15 +477,10 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
     __syncthreads();
   }
 
-  if constexpr (MODE == 1)
-    store_fc2<kRT, kStreamOut>(acc, target, reinterpret_cast<float*>(&stage[0][0]), n_rows, n0, lane, wave, row16, group, out_f32);
-  else
-    store_fc1<kRT>(acc, target, amax_part, out_cols, n0, tile, wave, row16, group, out_codes, out_scales);
+  store_fc1<kRT>(acc, target, amax_part, out_cols, n0, tile, wave, row16, group, out_codes, out_scales);
 }
 
-// Launches that stream more weights than they compute (few routes per
-// expert): see grouped_sparse_kernel.
-struct SparseArgs {
+struct ItemArgs {
   const uint8_t* w;
   const float* ws;
   int n_rows, out_cols;
@@ -536,7 +500,7 @@ struct SparseArgs {
 };
 
 // One workgroup's work, all wave-uniform.
-struct SparseItem {
+struct WorkItem {
   const uint8_t* w;  // the expert's weights and block scales
   const float* ws;
   int first, routes, tile;
@@ -544,27 +508,29 @@ struct SparseItem {
 };
 
 template <int KB, int MODE>
-struct SparseLds {
+struct ItemLds {
   __attribute__((aligned(16))) uint8_t stage[2][kGgRoutes * kGgStride];
   float a_scale[KB][kGgRoutes];
   int target[kGgRoutes];  // FC1: sorted position, FC2: pair; -1 = no route
   float amax_part[MODE == 0 ? kGgWaves : 1][kGgRoutes];
 };
 
-// One work item of the sparse kernel at kRT 16-route tiles (routes <= 16
-// kRT).  kDepth K blocks of weights are in flight (each reloads the
-// registers of the block just multiplied), and as many of staged activations
-// (one for kRT > 4, whose accumulators need the registers).  The MFMAs, the
-// scale products and their order are those of grouped_gemm_kernel, so the
-// results are bit-identical.
-template <int KB, int MODE, bool kPacked, bool kStreamOut, int kRT, int kDepth>
-__device__ __forceinline__ void sparse_item(const SparseArgs& a, const SparseItem& item,
-                                            SparseLds<KB, MODE>& lds) {
+// One work item at kRT 16-route tiles (routes <= 16 kRT).  kDepth: registers
+// for that many K blocks of weights; a block reloads the registers of the one
+// just multiplied (kSpread: of the one before, its loads between the MFMAs).
+// Activations take as many (one for kRT > 4, whose accumulators need the
+// registers).  K blocks in ascending order, one rescale per MFMA: the sums
+// are the same in every body.
+template <int KB, int MODE, bool kPacked, bool kStreamOut, bool kSparse, int kRT, int kDepth>
+__device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& item, ItemLds<KB, MODE>& lds) {
   constexpr int K = KB * kGroup;
   constexpr int kR = 16 * kRT;
   constexpr int kStage = kR * kGgStride;
   constexpr int kD = kDepth < KB ? kDepth : KB;             // K blocks in flight
   constexpr int kA = kRT > 4 ? 1 : kD;                       // K blocks of activations in registers
+  // Contraction-sized items of dense batches: the next block's loads go out
+  // between the MFMAs.
+  constexpr bool kSpread = !kSparse && kRT > 4;
   constexpr int kStaged = kR * kGroup / (16 * kGgThreads);  // 16-byte copies per thread and K block
   static_assert(kStaged >= 1, "at least 32 routes: one copy per thread and K block");
   const int n_rows = a.n_rows, out_cols = a.out_cols, top_k = a.top_k;
@@ -609,26 +575,30 @@ __device__ __forceinline__ void sparse_item(const SparseArgs& a, const SparseIte
       const_cast<uint8_t*>(wexp), 0, static_cast<uint32_t>(n_rows) * K, 0x00020000);
   const uint32_t w_lane = kPacked ? lane * 16 : row16 * K + group * 16;
   int32x8 wf[kD][kGgWaveTiles];
-  constexpr int kStreamed = kPacked ? 2 : 0;  // non-temporal: most experts have this item only
+  // Sparse batches read the weights non-temporally (most experts have this
+  // item only); otherwise an expert's next item finds them in the L2.
+  constexpr int kStreamed = kSparse && kPacked ? 2 : 0;
+  auto load_tile = [&](int kb, int t) {
+    const uint32_t base = static_cast<uint32_t>(tile_row(t)) * K;
+    int32x4 lo, hi;
+    if constexpr (kPacked) {
+      lo = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * 2048, kStreamed);
+      hi = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * 2048 + 1024, kStreamed);
+    } else {
+      lo = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * kGroup, kStreamed);
+      hi = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * kGroup + 64, kStreamed);
+    }
+    int32x8 v;
+    v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
+    v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
+    wf[kb % kD][t] = v;
+  };
   auto load_weights = [&](int kb) {
 #pragma unroll
-    for (int t = 0; t < kGgWaveTiles; ++t) {
-      const uint32_t base = static_cast<uint32_t>(tile_row(t)) * K;
-      int32x4 lo, hi;
-      if constexpr (kPacked) {
-        lo = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * 2048, kStreamed);
-        hi = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * 2048 + 1024, kStreamed);
-      } else {
-        lo = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * kGroup, kStreamed);
-        hi = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_lane, base + kb * kGroup + 64, kStreamed);
-      }
-      int32x8 v;
-      v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
-      v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
-      wf[kb % kD][t] = v;
-    }
+    for (int t = 0; t < kGgWaveTiles; ++t) load_tile(kb, t);
   };
-  constexpr int kEarly = (kD + 1) / 2;  // weight blocks issued before the activations
+  constexpr int kEarly = (kD + 1) / 2;        // weight blocks issued before the activations
+  constexpr int kAhead = kSpread ? 1 : kD;    // and before the first MFMA
 #pragma unroll
   for (int kb = 0; kb < kEarly; ++kb) load_weights(kb);
   __builtin_amdgcn_sched_barrier(0);
@@ -663,7 +633,7 @@ __device__ __forceinline__ void sparse_item(const SparseArgs& a, const SparseIte
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int kb = kEarly; kb < kD; ++kb) load_weights(kb);
+  for (int kb = kEarly; kb < kAhead; ++kb) load_weights(kb);
   float w_rows[2][KB];
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
@@ -685,36 +655,85 @@ __device__ __forceinline__ void sparse_item(const SparseArgs& a, const SparseIte
   for (int t = 0; t < kGgWaveTiles; ++t)
 #pragma unroll
     for (int rt = 0; rt < kRT; ++rt) acc[t][rt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (kSpread) {
+    // The next block's activation copies, then one weight tile (two loads)
+    // per unit, spread over the route tiles: issued in one go they hold the
+    // wave's MFMAs back while the memory pipeline drains.  The scale FMAs of
+    // a route tile follow the next one's MFMAs.
+    constexpr int kUnits = kStaged + kGgWaveTiles;
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (kA == 1) {
-      if (kb + 1 < KB) stage_load(kb + 1);
+    for (int kb = 0; kb < KB; ++kb) {
       __builtin_amdgcn_sched_barrier(0);
-    }
-    const uint8_t* buf = stage + (kb & 1) * kStage;
+      const uint8_t* buf = stage + (kb & 1) * kStage;
+      floatx4 partial[2][kGgWaveTiles];
+      float as_prev = 0.0f;
 #pragma unroll
-    for (int rt = 0; rt < kRT; ++rt) {
-      const int route = 16 * rt + row16;
-      const int32x8 bfrag = load_fragment(buf + route * kGgStride, 0, group);
-      const float as = lds.a_scale[kb][route];
+      for (int rt = 0; rt <= kRT; ++rt) {
+        if (kb + 1 < KB) {  // units rt (and, on the last route tile, the rest)
 #pragma unroll
-      for (int t = 0; t < kGgWaveTiles; ++t) {
-        const floatx4 partial = mfma_fp8(wf[kb % kD][t], bfrag);
-        scale_accumulate(acc[t][rt], partial, w_rows[t < 2 ? 0 : 1][kb] * as);
-        asm volatile("" : "+v"(acc[t][rt]));
+          for (int u = 0; u < kUnits; ++u) {
+            if (u != rt && !(rt == kRT - 1 && u >= kRT)) continue;
+            if (u < kStaged)
+              staged[0][u] = view.load16(src[u] + (kb + 1) * kGroup);
+            else
+              load_tile(kb + 1, u - kStaged);
+          }
+        }
+        float as = 0.0f;
+        if (rt < kRT) {
+          const int route = 16 * rt + row16;
+          const int32x8 bfrag = load_fragment(buf + route * kGgStride, 0, group);
+          as = lds.a_scale[kb][route];
+#pragma unroll
+          for (int t = 0; t < kGgWaveTiles; ++t) partial[rt & 1][t] = mfma_fp8(wf[kb % kD][t], bfrag);
+        }
+        if (rt > 0) {
+#pragma unroll
+          for (int t = 0; t < kGgWaveTiles; ++t) {
+            scale_accumulate(acc[t][rt - 1], partial[(rt - 1) & 1][t], w_rows[t < 2 ? 0 : 1][kb] * as_prev);
+            // Materialise the sum here: the accumulators are only used under
+            // the epilogue's per-route conditions, and without this the
+            // compiler sinks every K block's FMAs (all products stay live).
+            asm volatile("" : "+v"(acc[t][rt - 1]));
+          }
+        }
+        as_prev = as;
+        __builtin_amdgcn_sched_barrier(0);
       }
+      if (kb + 1 < KB) stage_store(kb + 1);
+      lds_barrier();
     }
-    __builtin_amdgcn_sched_barrier(0);
-    if (kb + kD < KB) {  // into the registers this block has just left
-      if constexpr (kA > 1) stage_load(kb + kD);
-      load_weights(kb + kD);
+  } else {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kA == 1) {
+        if (kb + 1 < KB) stage_load(kb + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const uint8_t* buf = stage + (kb & 1) * kStage;
+#pragma unroll
+      for (int rt = 0; rt < kRT; ++rt) {
+        const int route = 16 * rt + row16;
+        const int32x8 bfrag = load_fragment(buf + route * kGgStride, 0, group);
+        const float as = lds.a_scale[kb][route];
+#pragma unroll
+        for (int t = 0; t < kGgWaveTiles; ++t) {
+          const floatx4 partial = mfma_fp8(wf[kb % kD][t], bfrag);
+          scale_accumulate(acc[t][rt], partial, w_rows[t < 2 ? 0 : 1][kb] * as);
+          asm volatile("" : "+v"(acc[t][rt]));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (kb + kD < KB) {  // into the registers this block has just left
+        if constexpr (kA > 1) stage_load(kb + kD);
+        load_weights(kb + kD);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (kb + 1 < KB) stage_store(kb + 1);
+      lds_barrier();
     }
-    __builtin_amdgcn_sched_barrier(0);
-    if (kb + 1 < KB) stage_store(kb + 1);
-    lds_barrier();
   }
-
 
   if constexpr (MODE == 1)
     store_fc2<kRT, kStreamOut>(acc, lds.target, reinterpret_cast<float*>(stage), n_rows, n0, lane, wave, row16, group, a.out_f32);
@@ -722,33 +741,43 @@ __device__ __forceinline__ void sparse_item(const SparseArgs& a, const SparseIte
     store_fc1<kRT>(acc, lds.target, lds.amax_part, out_cols, n0, tile, wave, row16, group, a.out_codes, a.out_scales);
 }
 
-// The GEMMs of sparse batches (at most kSparseRoutes routes per expert on
-// average): bound by the weight stream, each expert's weights being read
-// once, by its one work item.  grouped_gemm_kernel spends its registers on
-// 128 accumulators and has one K block in flight; here the workgroup picks
-// the smallest of four bodies that holds its item (32, 64, 96 or 128 routes)
-// and the registers go to weights in flight, read non-temporally.  Measured
-// (E256 H2048 I512, FC1 / FC2 us, kernel trace, one box): 131 rows (4 routes
-// per expert) 104.8 / 61.8 -> 87.6 / 46.1 (6.1 / 6.0 TB/s), 517 rows of an
-// uneven router 92.0 / 60.2 -> 84.1 / 48.4, 2048 rows (64 per expert) 117.3 /
-// 84.0 -> 106.6 / 78.6; non-temporal loads are half of the gain.  Two more
-// depths were tried (2 and 4 to 5 blocks for the 32-route body): within 1 us,
-// 5 spills.  At 128 routes per expert (4,096 rows) it is slower (144 / 118 ->
-// 152 / 118 us cached, 165 / 126 us non-temporal): the matrix work then wants
-// the loads spread between the MFMAs and the experts' second items the
-// weights in L2.
-template <int KB, int MODE, bool kPacked, bool kStreamOut>
-__global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2))) void grouped_sparse_kernel(
-    SparseArgs a) {
+// The grouped GEMMs over sorted items.
+//
+// kSparse: batches of at most kSparseRoutes routes per expert on average.
+// They are bound by the weight stream, each expert's weights being read once,
+// by its one work item: registers go to weights in flight in every body, read
+// non-temporally.  Measured against a kernel of the 128-route body alone, one
+// cached K block in flight (E256 H2048 I512, FC1 / FC2 us, kernel trace, one
+// box): 131 rows (4 routes per expert) 104.8 / 61.8 -> 87.6 / 46.1 (6.1 / 6.0
+// TB/s), 517 rows of an uneven router 92.0 / 60.2 -> 84.1 / 48.4, 2048 rows
+// (64 per expert) 117.3 / 84.0 -> 106.6 / 78.6; non-temporal loads are half
+// of the gain.  Other depths (2 and 4 blocks for the 32-route body) are
+// within 1 us, 5 spills.
+//
+// Otherwise an expert has more than one item, which share its weights in the
+// L2 (cached loads; non-temporal 145 -> 157 us for FC1 at 4,096 rows), and the
+// matrix work of its full items wants the loads spread between the MFMAs; its
+// last item is often partial and takes a smaller body.  Against the 128-route
+// body for every item (same box, FC1 / FC2 us): 3,668 rows E128 I768 with the
+// shared expert 172.4 / 122.5 -> 161.6 / 115.1, 4,096 rows E256 I512 145.4 /
+// 119.5 -> 144.7 / 110.9, 2,500 rows E128 137.2 / 94.7 -> 131.3 / 90.7, 140
+// rows E16 H1024 I256 15.7 / 7.8 -> 13.8 / 6.5.  Bound: about half by waiting
+// for the K blocks' loads (one block ahead is what the accumulators leave),
+// the rest MFMAs and their rescale in turn.  64-route items at three waves per
+// SIMD were slower (165 -> 185 us: more weight traffic per MFMA), three weight
+// blocks for the 96-route body equal.
+template <int KB, int MODE, bool kPacked, bool kStreamOut, bool kSparse>
+__global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2))) void grouped_items_kernel(
+    ItemArgs a) {
   constexpr int K = KB * kGroup;
-  __shared__ SparseLds<KB, MODE> lds;
-  // Workgroups to (item, tile) as in grouped_gemm_kernel.
+  __shared__ ItemLds<KB, MODE> lds;
+  // XCD-aware order, as in grouped_by_pair_kernel.
   const int b = blockIdx.x;
   const int xcd = b % kGgXcds, j = b / kGgXcds;
   const int logical = ((j / a.chunk) * kGgXcds + xcd) * a.chunk + j % a.chunk;
   const int within = logical % a.chunk;
   const int item_index = (logical / a.chunk) * 2 + (within & 1);
-  SparseItem item;
+  WorkItem item;
   item.tile = within >> 1;
   item.dense = item_index >= a.max_items;
   if (!item.dense) {
@@ -768,13 +797,13 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
     item.ws = a.shared.ws;
   }
   if (item.routes <= 32)
-    sparse_item<KB, MODE, kPacked, kStreamOut, 2, 3>(a, item, lds);
+    item_body<KB, MODE, kPacked, kStreamOut, kSparse, 2, 3>(a, item, lds);
   else if (item.routes <= 64)
-    sparse_item<KB, MODE, kPacked, kStreamOut, 4, 3>(a, item, lds);
+    item_body<KB, MODE, kPacked, kStreamOut, kSparse, 4, 3>(a, item, lds);
   else if (item.routes <= 96)
-    sparse_item<KB, MODE, kPacked, kStreamOut, 6, 2>(a, item, lds);
+    item_body<KB, MODE, kPacked, kStreamOut, kSparse, 6, 2>(a, item, lds);
   else
-    sparse_item<KB, MODE, kPacked, kStreamOut, 8, 2>(a, item, lds);
+    item_body<KB, MODE, kPacked, kStreamOut, kSparse, 8, 2>(a, item, lds);
 }
 
 struct GroupedLaunch {
@@ -819,53 +848,41 @@ void launch_grouped(const GroupedLaunch& g, hipStream_t s) {
   // prefill batch (29k routes, 240 MB of rows) is 10 us slower that way.
   const bool stream_out =
       MODE == 1 && (static_cast<int64_t>(g.max_items) + shared_items) * kGgRoutes <= kStreamOutRoutes;
-  if (g.sparse && logical >= kResidentGroups) {
-    const SparseArgs a{g.w, g.ws, g.n_rows, g.out_cols, g.a, g.a_bytes, g.as, g.sorted_ids, g.top_k, g.items,
-                       g.num_items, g.max_items, g.shared, n_tiles, chunk, g.codes, g.scales, g.out};
-    const bool packed = g.layout == D3_LAYOUT_FRAGMENT;
-    if constexpr (MODE == 1) {
-      if (stream_out) {
-        if (packed)
-          hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, true, true>), dim3(blocks), dim3(kGgThreads), 0, s, a);
-        else
-          hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, false, true>), dim3(blocks), dim3(kGgThreads), 0, s, a);
-        return;
-      }
-    }
-    if (packed)
-      hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, true, false>), dim3(blocks), dim3(kGgThreads), 0, s, a);
-    else
-      hipLaunchKernelGGL((grouped_sparse_kernel<KB, MODE, false, false>), dim3(blocks), dim3(kGgThreads), 0, s, a);
-    return;
-  }
-#define D3_GG_ARGS dim3(blocks), dim3(kGgThreads), 0, s, g.w, g.ws, g.n_rows, g.out_cols, g.a, \
-                   g.a_bytes, g.as, g.sorted_ids, g.top_k, g.items, g.num_items, g.max_items, \
-                   g.shared, n_tiles, chunk, g.parts, g.capacity, g.list_ids, g.list_items,   \
-                   g.list_count, g.codes, g.scales, g.out
+  const bool packed = g.layout == D3_LAYOUT_FRAGMENT;
+  const dim3 grid(blocks), block(kGgThreads);
   if constexpr (MODE == 0) {
     if (g.parts > 0) {
-      if (g.layout == D3_LAYOUT_FRAGMENT)
-        hipLaunchKernelGGL((grouped_gemm_kernel<KB, MODE, true, true>), D3_GG_ARGS);
+#define D3_GG_ARGS                                                                                         \
+  grid, block, 0, s, g.w, g.ws, g.n_rows, g.out_cols, g.a, g.a_bytes, g.as, g.sorted_ids, g.top_k, g.num_items, \
+      g.max_items, n_tiles, chunk, g.parts, g.capacity, g.list_ids, g.list_items, g.list_count, g.codes, g.scales
+      if (packed)
+        hipLaunchKernelGGL((grouped_by_pair_kernel<KB, true>), D3_GG_ARGS);
       else
-        hipLaunchKernelGGL((grouped_gemm_kernel<KB, MODE, false, true>), D3_GG_ARGS);
+        hipLaunchKernelGGL((grouped_by_pair_kernel<KB, false>), D3_GG_ARGS);
+#undef D3_GG_ARGS
       return;
     }
   }
+  const ItemArgs a{g.w, g.ws, g.n_rows, g.out_cols, g.a, g.a_bytes, g.as, g.sorted_ids, g.top_k, g.items,
+                   g.num_items, g.max_items, g.shared, n_tiles, chunk, g.codes, g.scales, g.out};
+  const bool sparse = g.sparse && logical >= kResidentGroups;
+#define D3_ITEMS(STREAM)                                                                               \
+  if (packed && sparse)                                                                               \
+    hipLaunchKernelGGL((grouped_items_kernel<KB, MODE, true, STREAM, true>), grid, block, 0, s, a);   \
+  else if (packed)                                                                                    \
+    hipLaunchKernelGGL((grouped_items_kernel<KB, MODE, true, STREAM, false>), grid, block, 0, s, a);  \
+  else if (sparse)                                                                                    \
+    hipLaunchKernelGGL((grouped_items_kernel<KB, MODE, false, STREAM, true>), grid, block, 0, s, a);  \
+  else                                                                                                \
+    hipLaunchKernelGGL((grouped_items_kernel<KB, MODE, false, STREAM, false>), grid, block, 0, s, a);
   if constexpr (MODE == 1) {
     if (stream_out) {
-      if (g.layout == D3_LAYOUT_FRAGMENT)
-        hipLaunchKernelGGL((grouped_gemm_kernel<KB, MODE, true, false, true>), D3_GG_ARGS);
-      else
-        hipLaunchKernelGGL((grouped_gemm_kernel<KB, MODE, false, false, true>), D3_GG_ARGS);
+      D3_ITEMS(true)
       return;
     }
   }
-  if (g.layout == D3_LAYOUT_FRAGMENT) {
-    hipLaunchKernelGGL((grouped_gemm_kernel<KB, MODE, true, false>), D3_GG_ARGS);
-  } else {
-    hipLaunchKernelGGL((grouped_gemm_kernel<KB, MODE, false, false>), D3_GG_ARGS);
-  }
-#undef D3_GG_ARGS
+  D3_ITEMS(false)
+#undef D3_ITEMS
 }
 
 template <int MODE>
