@@ -117,14 +117,18 @@ def sortless_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
     -> 126 us, 256 rows 221 -> 140 us; E256 256 rows 160 us either way; E128
     100 rows, 6 per expert, 112 against 122 us).  With few experts their
     route slices run side by side instead (E16: 26 against 42 us)."""
-    lib = _lib.load()
-    shapes = (hidden // 128 in (8, 16) and intermediate // 128 in (2, 4, 6, 8)
-              and hidden % 128 == 0 and intermediate % 128 == 0
-              and hidden % lib.d3_expert_tile_rows(intermediate) == 0)
     pairs = rows * top_k
     busy = rows > 64 and num_experts >= 64 and pairs >= 8 * num_experts
-    return (shapes and rows <= 256 and top_k <= 8 and not busy
+    return (sortless_covers(rows, hidden, intermediate, top_k) and not busy
             and (pairs >= num_experts or pairs <= SORTLESS_PAIRS))
+
+
+def sortless_covers(rows: int, hidden: int, intermediate: int, top_k: int = 8) -> bool:
+    """Whether the expert GEMMs without a route sort are compiled for a batch."""
+    return (hidden // 128 in (8, 16) and intermediate // 128 in (2, 4, 6, 8)
+            and hidden % 128 == 0 and intermediate % 128 == 0
+            and hidden % _lib.load().d3_expert_tile_rows(intermediate) == 0
+            and rows <= 256 and top_k <= 8)
 
 
 def fragment_weights(experts) -> bool:
@@ -712,14 +716,17 @@ class DecodeStep:
         # and the batch suit them (sortless_suited).  Measured at 64 slots:
         # E128 (8 routes per expert) and the reference model's E256 / I512 (2
         # per expert: 127 us against 134 us for the sorted chain).
-        suited = sortless_suited(slots, num_experts, hidden, intermediate, top_k)
+        # A caller who asks for the three-launch step gets the sortless chain
+        # wherever it covers the slots and their routes could reach every expert.
+        reach = slots * top_k >= num_experts
         if sortless is None:
-            sortless = suited
+            sortless = (reach and sortless_covers(slots, hidden, intermediate, top_k) if frontless
+                        else sortless_suited(slots, num_experts, hidden, intermediate, top_k))
         self.sortless = bool(sortless)
         # The FC1 from the slots has a workgroup per expert, which pays when the
         # slots' routes reach most of them.
         if frontless is None:
-            frontless = self.sortless and slots * top_k >= num_experts
+            frontless = self.sortless and reach
         self.frontless = bool(frontless)
         if self.frontless and not self.sortless:
             raise ValueError("frontless runs the sortless chain (sortless=True)")

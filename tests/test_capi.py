@@ -318,3 +318,22 @@ def test_packed_operands_follow_their_source_tensor():
     assert ew.fc2_operands(ex)[2] == ew.LAYOUT_REFERENCE
     ex.w13_weight = ex.w13_weight.clone()
     assert ew.fc1_operands(ex)[2] == ew.LAYOUT_REFERENCE
+
+
+@pytest.mark.parametrize("slots,experts,sortless",
+                         [(64, 128, True), (128, 128, False), (256, 128, False), (256, 16, True),
+                          (16, 256, True), (64, 4096, False)])
+def test_decode_step_default_chains(slots, experts, sortless):
+    """The chain a DecodeStep takes by default, and that asking for the
+    three-launch step is answered alike whichever chain the default is: taken
+    where the slots' routes could reach every expert, refused below."""
+    from drama3_amd.pipeline import DecodeStep
+
+    step = DecodeStep(slots, experts, 1024, 256, device="cpu")
+    assert step.sortless == sortless and step.frontless == (sortless and slots * 8 >= experts)
+    if slots * 8 >= experts:
+        asked = DecodeStep(slots, experts, 1024, 256, device="cpu", frontless=True)
+        assert asked.frontless and asked.sortless
+    else:
+        with pytest.raises(ValueError):
+            DecodeStep(slots, experts, 1024, 256, device="cpu", frontless=True)
