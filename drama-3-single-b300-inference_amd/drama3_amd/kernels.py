@@ -16,7 +16,7 @@ from . import _lib
 from ._lib import call, ptr
 from .pipeline import (SORTLESS_PAIRS, WIDE_SORT_PAIRS, MoEWorkspace, Shape, by_pair_suited,
                        dtype_code, fragment_weights, grouped_supported, require_cuda,
-                       sortless_suited)
+                       rows_in_view, sortless_suited)
 
 TOP_K = 8
 # Most rows of routed_moe without a route sort (no expert has more routes than
@@ -121,7 +121,7 @@ def _routed(x, topk_ids, topk_weights, experts, block_m: int = 16):
     if x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
     if (rows * top_k <= SORTLESS_PAIRS and sortless_suited(rows, e, h, i, top_k)
-            and fragment_weights(experts)):
+            and rows_in_view(x) and fragment_weights(experts)):
         return ws.small_forward(x, ids, weights, experts, out)
     return ws.experts_forward(x, ids, weights, experts, out=out)
 

@@ -131,6 +131,12 @@ def sortless_covers(rows: int, hidden: int, intermediate: int, top_k: int = 8) -
             and rows <= 256 and top_k <= 8)
 
 
+def rows_in_view(x: torch.Tensor) -> bool:
+    """Whether the rows span less than the 2 GiB that a kernel's buffer view
+    of them covers (the route sort's chain reads rows of any stride)."""
+    return x.shape[0] * x.stride(0) * x.element_size() < 1 << 31
+
+
 def fragment_weights(experts) -> bool:
     """Whether both weight tensors have fragment-major copies."""
     return (fc1_operands(experts)[2] == LAYOUT_FRAGMENT

@@ -376,3 +376,22 @@ def test_few_slots_match_sorted_chain(device, slots, live):
         step(occupancy.to(device), xs, ls, packed)
     torch.cuda.synchronize()
     assert compare(few, chain) == live
+
+
+def test_small_moe_rows_far_apart(device):
+    """Rows that span 2 GiB and more run as packed rows do."""
+    from drama3_amd.expert_weights import prepare_experts
+    from drama3_amd.kernels import small_batch_moe
+    from drama3_amd.workloads import make_experts
+
+    gen = torch.Generator("cpu").manual_seed(41)
+    rows, h = 2, 1024
+    packed = prepare_experts(make_experts(gen, 256, h, 256).to(device))
+    x = torch.randn((rows, h), generator=gen).to(torch.bfloat16).to(device)
+    ids = torch.stack([torch.randperm(256, generator=gen)[:8] for _ in range(rows)]).to(device)
+    weights = torch.rand((rows, 8), generator=gen).to(device)
+    stride = 1 << 29
+    far = torch.empty(stride + h, dtype=torch.bfloat16, device=device).as_strided((rows, h), (stride, 1))
+    far.copy_(x)
+    got, expected = (small_batch_moe(t, ids, weights, packed) for t in (far, x))
+    assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
