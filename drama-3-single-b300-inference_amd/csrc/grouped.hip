@@ -748,7 +748,7 @@ __device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& ite
 // by its one work item: registers go to weights in flight in every body, read
 // non-temporally.  Measured against a kernel of the 128-route body alone, one
 // cached K block in flight (E256 H2048 I512, FC1 / FC2 us, kernel trace, one
-// box): 131 rows (4 routes per expert) 104.8 / 61.8 -> 87.6 / 46.1 (6.1 / 6.0
+// card): 131 rows (4 routes per expert) 104.8 / 61.8 -> 87.6 / 46.1 (6.1 / 6.0
 // TB/s), 517 rows of an uneven router 92.0 / 60.2 -> 84.1 / 48.4, 2048 rows
 // (64 per expert) 117.3 / 84.0 -> 106.6 / 78.6; non-temporal loads are half
 // of the gain.  Other depths (2 and 4 blocks for the 32-route body) are
@@ -758,7 +758,7 @@ __device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& ite
 // L2 (cached loads; non-temporal 145 -> 157 us for FC1 at 4,096 rows), and the
 // matrix work of its full items wants the loads spread between the MFMAs; its
 // last item is often partial and takes a smaller body.  Against the 128-route
-// body for every item (same box, FC1 / FC2 us): 3,668 rows E128 I768 with the
+// body for every item (same card, FC1 / FC2 us): 3,668 rows E128 I768 with the
 // shared expert 172.4 / 122.5 -> 161.6 / 115.1, 4,096 rows E256 I512 145.4 /
 // 119.5 -> 144.7 / 110.9, 2,500 rows E128 137.2 / 94.7 -> 131.3 / 90.7, 140
 // rows E16 H1024 I256 15.7 / 7.8 -> 13.8 / 6.5.  Bound: about half by waiting
