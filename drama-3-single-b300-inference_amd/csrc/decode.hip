@@ -18,12 +18,14 @@
 //
 // A workgroup whose expert receives no route exits after its first weight
 // loads (those bytes are wasted): the layout suits batches whose routes
-// cover most experts.  A handful of rows over many experts (fewer routes
-// than experts, at most 256) takes the pair grid instead: a workgroup per
-// (pair, row tile), whose expert is the pair's; it goes on only if no
-// earlier pair names that expert, and then takes all of the expert's pairs.
-// Every wave holds all the ids (four per lane), so that is decided from four
-// ballots without LDS, and no weight is issued for an expert without routes.
+// cover most experts.  A handful of rows (at most 256 pairs) takes the pair
+// grid instead: a workgroup per (pair, row tile), whose expert is the pair's;
+// it goes on only if the pair is the first of one of its expert's 16-route
+// tiles, and then takes that tile.  Every wave holds all the ids (four per
+// lane), so that is decided from four ballots without LDS, no weight is
+// issued for an expert without routes, and a busy expert's route tiles run
+// side by side (E256 H2048 I512, all 128 pairs of 16 rows on one expert: 101
+// us with one workgroup walking the tiles, 39 us so, 36 us on a route sort).
 //
 // The FC1 can also start from the slots themselves (MODE 1), which removes
 // the front launch: slot s routes to expert e at rank c when c, the number
@@ -56,11 +58,10 @@ struct DecodeArgs {
   int capacity;  // slot rows
   int top_k;
   int exact_routes;
-  // MODE 0 / 2 / 3: routed ids of every row (32-bit words, id_words apart)
-  // and the live row count (front output, or none)
+  // MODE 0 / 2 / 3: routed ids of every row and the live row count (front
+  // output, or none); the pair grid reads them as 32-bit words, id_words apart
   const int32_t* ids;
   int id_words;
-  int row_routes;  // most routes of one expert in a row: 1 (router ids) or top_k (given ids)
   const int32_t* row_count;
   // MODE 0: q rows and their scales; MODE 2: bf16 gate|up by pair
   const void* act;
@@ -105,7 +106,7 @@ struct LogitPass {
 //         -> fp32 down by pair.
 // MODE 3: FC1 from given ids: x rows quantised while staged (as MODE 1) ->
 //         bf16 gate|up by pair.
-// kPairGrid (MODE 0, 2, 3): workgroups by (pair, weight tile).
+// kPairGrid (MODE 0, 2; MODE 3 always): workgroups by (pair, weight tile).
 // TILES weight tiles per workgroup, streamed through the registers in halves
 // (TILES > 1: routes beyond the first 16 reload the weight tiles).
 // PASSES (MODE 1): ranking passes of 64 slots the kernel is built for.
@@ -116,7 +117,7 @@ struct LogitPass {
 // (route slices): one weight tile per workgroup, except FC1 from the slots
 // at K = 2048, whose two bodies together would not fit the registers.
 constexpr bool from_x(int mode) { return mode == 1 || mode == 3; }  // FC1 quantises the x rows itself
-constexpr bool sliced_kernel(int kb, int mode, int tiles) { return tiles == 1 && !(from_x(mode) && kb >= 16); }
+constexpr bool sliced_kernel(int kb, int mode, int tiles) { return tiles == 1 && !(mode == 1 && kb >= 16); }
 
 // LDS of one decode GEMM workgroup (declared once in the kernel, shared by
 // both instantiations of its body).
@@ -139,7 +140,7 @@ struct DecodeLds {
 template <int KB, int RT, int MODE, int TILES, int PASSES, bool kWholeFirst, bool kEarly, bool kPairGrid = false>
 __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<KB, MODE>& lds, int unit,
                                                  int first_tile, int slice, int slices) {
-  static_assert(!kPairGrid || (MODE != 1 && kEarly), "the pair grid reads ids");
+  static_assert(kPairGrid ? MODE != 1 && kEarly : MODE != 3, "the pair grid reads ids; given ids take it");
   constexpr bool kFromX = from_x(MODE);
   const uint8_t* __restrict__ w = a.w;
   const float* __restrict__ ws = a.ws;
@@ -163,7 +164,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   auto& route_pairs = lds.route_pairs;
   auto& route_slots = lds.route_slots;
   auto& chunk_counts = lds.chunk_counts;
-  const int first_route = 16 * slice;  // this slice's first route tile
+  int first_route = 16 * slice;  // this slice's (pair grid: this pair's) first route tile
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int row16 = lane & 15;
@@ -188,16 +189,17 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
     const int pairs = live_rows(a.row_count, capacity) * top_k;
     expert = __builtin_amdgcn_readfirstlane(static_cast<int>(own));
     if (unit >= pairs || expert < 0 || expert >= a.num_experts) return;  // uniform
-    bool earlier = false;
+    int rank = 0;  // of this pair among the expert's
 #pragma unroll
     for (int c = 0; c < kPairGridPairs / kWave; ++c) {
       const int p = c * kWave + lane;
       pair_hits[c] = __ballot(p < pairs && static_cast<int>(pair_ids[c]) == expert);
       const int before = unit - c * kWave;  // pairs of this chunk before `unit`
       const uint64_t mask = before <= 0 ? 0ull : (before >= kWave ? ~0ull : (1ull << before) - 1ull);
-      earlier |= (pair_hits[c] & mask) != 0ull;
+      rank += __popcll(pair_hits[c] & mask);
     }
-    if (earlier) return;  // uniform: an earlier pair's workgroup has this expert
+    if (rank % 16 != 0) return;  // uniform: an earlier pair's workgroup has this pair's route tile
+    first_route = rank;
   }
   const uint8_t* wexp = w + static_cast<size_t>(expert) * n_rows * K;
   const float* wsexp = ws + static_cast<size_t>(expert) * (n_rows / kGroup) * KB;
@@ -389,16 +391,16 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   } else {
     // 1. The routed ids of every slot row (past the capacity: zeros, masked
     //    below), issued before any weight.
-    const uint32_t id_bytes = static_cast<uint32_t>(capacity * top_k * a.id_words) * 4;
+    const uint32_t id_bytes = static_cast<uint32_t>(capacity * top_k) * 4;
     const BufferView id_view(a.ids, id_bytes);
     uint32_t id[kIdsPerThread];
 #pragma unroll
     for (int j = 0; j < kIdsPerThread; ++j) {
-      const uint32_t p = static_cast<uint32_t>(j * kGemmThreads + threadIdx.x) * a.id_words;
+      const uint32_t p = static_cast<uint32_t>(j * kGemmThreads + threadIdx.x);
       id[j] = id_view.load4(p * 4 < id_bytes ? p * 4 : kNoRow);
     }
     const int rows = live_rows(a.row_count, capacity);
-    if (slice > 0 && first_route >= rows * a.row_routes) return;  // uniform
+    if (slice > 0 && first_route >= rows) return;  // at most one route per live row (uniform)
     // 2. The first half of the first weight tile streams meanwhile.
     if constexpr (kEarly) {
       load_weights(first_tile, 0, kWholeFirst ? KB : kFirstHalf);
@@ -427,12 +429,8 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
         base += w2 < wave ? c : 0;
         chunk_base += c;
       }
-      if ((hits[j] >> lane) & 1ull) {
-        const int r = base + __popcll(hits[j] & lanemask_lt());
-        const int pair = j * kGemmThreads + static_cast<int>(threadIdx.x);
-        route_pairs[r] = pair;
-        if constexpr (kFromX) route_slots[r] = pair / top_k;
-      }
+      if ((hits[j] >> lane) & 1ull)
+        route_pairs[base + __popcll(hits[j] & lanemask_lt())] = j * kGemmThreads + threadIdx.x;
     }
     routes = chunk_base;
   }
@@ -706,6 +704,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
     floatx4 acc[RT];
     mma(acc);
     epilogue(acc, first_tile);
+    if constexpr (kPairGrid) return;  // further route tiles are other pairs'
     for (int m0 = first_route + 16 * slices; m0 < routes; m0 += 16 * slices) {
       __syncthreads();  // previous route tile fully consumed
       fetch_tile(m0);
@@ -718,7 +717,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   }
 }
 
-template <int KB, int RT, int MODE, int TILES, int PASSES = 1, bool kWholeFirst = false, bool kPairGrid = false>
+template <int KB, int RT, int MODE, int TILES, int PASSES = 1, bool kWholeFirst = false>
 __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2))) void decode_gemm_kernel(
     DecodeArgs a) {
   __shared__ DecodeLds<KB, MODE> lds;
@@ -731,11 +730,6 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2)
   // weight tile in its L2.
   const int slices = sliced_kernel(KB, MODE, TILES) && a.slices > 1 ? a.slices : 1;
   int unit = static_cast<int>(blockIdx.x), slice = 0;
-  if constexpr (kPairGrid) {
-    decode_gemm_body<KB, RT, MODE, TILES, PASSES, kWholeFirst, true, true>(a, lds, unit / groups,
-                                                                          (unit % groups) * TILES, 0, 1);
-    return;
-  }
   if (slices > 1) {
     const int units = a.num_experts * groups;
     const int stride = (units + 7) / 8 * 8;
@@ -755,6 +749,15 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2)
     }
   }
   decode_gemm_body<KB, RT, MODE, TILES, PASSES, kWholeFirst, true>(a, lds, expert, first_tile, slice, slices);
+}
+
+// The pair grid: workgroup -> (pair, weight tile).
+template <int KB, int RT, int MODE>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2))) void pair_gemm_kernel(DecodeArgs a) {
+  __shared__ DecodeLds<KB, MODE> lds;
+  const int tiles = a.n_rows / (kGemmWaves * RT * 16);
+  const int unit = static_cast<int>(blockIdx.x) / tiles;
+  decode_gemm_body<KB, RT, MODE, 1, 1, false, true, true>(a, lds, unit, static_cast<int>(blockIdx.x) % tiles, 0, 1);
 }
 
 bool aligned(const void* p, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
@@ -816,24 +819,8 @@ int tiles_per_group(int num_experts, int tiles, int capacity, int top_k, int mod
   return 1;
 }
 
-// The pair grid: fewer pairs than experts, few enough for one workgroup's
-// ballots.
-bool pair_grid(int num_experts, int capacity, int top_k) {
-  return capacity * top_k <= kPairGridPairs && capacity * top_k < num_experts;
-}
-
 template <int KB, int MODE>
-void launch_decode(int num_experts, hipStream_t s, const DecodeArgs& a) {
-  const int tiles = a.n_rows / tile_rows_for(KB);
-  if constexpr (MODE != 1) {
-    if (pair_grid(num_experts, a.capacity, a.top_k)) {
-      DecodeArgs args = a;
-      args.slices = 1;
-      hipLaunchKernelGGL((decode_gemm_kernel<KB, rt_for(KB), MODE, 1, 1, false, true>),
-                         dim3(a.capacity * a.top_k * tiles), dim3(kGemmThreads), 0, s, args);
-      return;
-    }
-  }
+void launch_expert_grid(int num_experts, int tiles, hipStream_t s, const DecodeArgs& a) {
   const int t = tiles_per_group(num_experts, tiles, a.capacity, a.top_k, MODE);
   if constexpr (MODE != 2) {
     if (t == 6) {
@@ -849,6 +836,27 @@ void launch_decode(int num_experts, hipStream_t s, const DecodeArgs& a) {
     launch_tiles<KB, MODE, 2>(num_experts, s, a);
   else
     launch_tiles<KB, MODE, 1>(num_experts, s, a);
+}
+
+// The pair grid: few enough pairs for one workgroup's ballots, and fewer of
+// them than experts.
+bool pair_grid(int num_experts, int capacity, int top_k) {
+  return capacity * top_k <= kPairGridPairs && capacity * top_k < num_experts;
+}
+
+// by_pairs: on the pair grid whatever the number of experts (given ids, where
+// an expert may take every pair).
+template <int KB, int MODE>
+void launch_decode(int num_experts, hipStream_t s, const DecodeArgs& a, bool by_pairs) {
+  const int tiles = a.n_rows / tile_rows_for(KB);
+  if constexpr (MODE != 1) {
+    if (MODE == 3 || by_pairs || pair_grid(num_experts, a.capacity, a.top_k)) {
+      hipLaunchKernelGGL((pair_gemm_kernel<KB, rt_for(KB), MODE>), dim3(a.capacity * a.top_k * tiles),
+                         dim3(kGemmThreads), 0, s, a);
+      return;
+    }
+  }
+  if constexpr (MODE != 3) launch_expert_grid<KB, MODE>(num_experts, tiles, s, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -1025,6 +1033,7 @@ struct GemmLaunch {
   int kb;
   int num_experts;
   DecodeArgs args;
+  bool by_pairs = false;
 };
 
 int check_expert_gemm(int32_t mode, const uint8_t* w, const float* ws, int32_t num_experts,
@@ -1059,7 +1068,6 @@ int check_expert_gemm(int32_t mode, const uint8_t* w, const float* ws, int32_t n
   args.num_experts = num_experts;
   args.ids = ids;
   args.id_words = 1;
-  args.row_routes = 1;
   args.row_count = row_count;
   args.act = a;
   args.act_scales = a_scales;
@@ -1072,19 +1080,19 @@ int check_expert_gemm(int32_t mode, const uint8_t* w, const float* ws, int32_t n
 
 void launch_expert_gemm(const GemmLaunch& l, hipStream_t s) {
   if (l.mode == 0) {
-    if (l.kb == 8) launch_decode<8, 0>(l.num_experts, s, l.args);
-    else launch_decode<16, 0>(l.num_experts, s, l.args);
+    if (l.kb == 8) launch_decode<8, 0>(l.num_experts, s, l.args, l.by_pairs);
+    else launch_decode<16, 0>(l.num_experts, s, l.args, l.by_pairs);
   } else if (l.mode == 3) {
-    if (l.kb == 8) launch_decode<8, 3>(l.num_experts, s, l.args);
-    else launch_decode<16, 3>(l.num_experts, s, l.args);
+    if (l.kb == 8) launch_decode<8, 3>(l.num_experts, s, l.args, l.by_pairs);
+    else launch_decode<16, 3>(l.num_experts, s, l.args, l.by_pairs);
   } else if (l.mode == 1) {
-    if (l.kb == 8) launch_decode<8, 1>(l.num_experts, s, l.args);
-    else launch_decode<16, 1>(l.num_experts, s, l.args);
+    if (l.kb == 8) launch_decode<8, 1>(l.num_experts, s, l.args, l.by_pairs);
+    else launch_decode<16, 1>(l.num_experts, s, l.args, l.by_pairs);
   } else {
-    if (l.kb == 2) launch_decode<2, 2>(l.num_experts, s, l.args);
-    else if (l.kb == 4) launch_decode<4, 2>(l.num_experts, s, l.args);
-    else if (l.kb == 6) launch_decode<6, 2>(l.num_experts, s, l.args);
-    else launch_decode<8, 2>(l.num_experts, s, l.args);
+    if (l.kb == 2) launch_decode<2, 2>(l.num_experts, s, l.args, l.by_pairs);
+    else if (l.kb == 4) launch_decode<4, 2>(l.num_experts, s, l.args, l.by_pairs);
+    else if (l.kb == 6) launch_decode<6, 2>(l.num_experts, s, l.args, l.by_pairs);
+    else launch_decode<8, 2>(l.num_experts, s, l.args, l.by_pairs);
   }
 }
 
@@ -1168,11 +1176,10 @@ int check_ids_fc1(const uint8_t* w, const float* ws, int32_t num_experts, int32_
   args.num_experts = num_experts;
   args.ids = static_cast<const int32_t*>(ids);
   args.id_words = ids_dtype == D3_DTYPE_I64 ? 2 : 1;
-  args.row_routes = top_k;
   args.x = x;
   args.x_stride = x_stride;
   args.out_bf16 = gate_up;
-  *launch = GemmLaunch{3, kb, num_experts, args};
+  *launch = GemmLaunch{3, kb, num_experts, args, true};
   return D3_OK;
 }
 
@@ -1359,7 +1366,7 @@ extern "C" int d3_small_moe(const uint8_t* w13, const float* s13, const uint8_t*
                              top_k, gate_up, nullptr, kPairGridPairs, nullptr, down, &fc2);
   if (status != D3_OK) return status;
   fc2.args.id_words = fc1.args.id_words;
-  fc2.args.row_routes = top_k;
+  fc2.by_pairs = true;
   hipStream_t s = as_stream(stream);
   launch_expert_gemm(fc1, s);
   launch_expert_gemm(fc2, s);

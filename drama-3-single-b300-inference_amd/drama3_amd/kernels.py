@@ -14,9 +14,9 @@ import torch
 
 from . import _lib
 from ._lib import call, ptr
-from .pipeline import (SORTLESS_PAIRS, WIDE_SORT_PAIRS, MoEWorkspace, Shape, by_pair_suited,
+from .pipeline import (WIDE_SORT_PAIRS, MoEWorkspace, Shape, by_pair_suited,
                        dtype_code, fragment_weights, grouped_supported, require_cuda,
-                       rows_in_view, sortless_suited)
+                       rows_in_view, small_suited, sortless_suited)
 
 TOP_K = 8
 # Most rows of routed_moe without a route sort (no expert has more routes than
@@ -120,8 +120,8 @@ def _routed(x, topk_ids, topk_weights, experts, block_m: int = 16):
     ids, weights = topk_ids.contiguous(), topk_weights.contiguous()
     if x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
-    if (rows * top_k <= SORTLESS_PAIRS and sortless_suited(rows, e, h, i, top_k)
-            and rows_in_view(x) and fragment_weights(experts)):
+    if (small_suited(rows, e, h, i, top_k) and rows_in_view(x)
+            and fragment_weights(experts)):
         return ws.small_forward(x, ids, weights, experts, out)
     return ws.experts_forward(x, ids, weights, experts, out=out)
 

@@ -131,6 +131,22 @@ def sortless_covers(rows: int, hidden: int, intermediate: int, top_k: int = 8) -
             and rows <= 256 and top_k <= 8)
 
 
+def small_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
+                 top_k: int = 8) -> bool:
+    """Whether d3_small_moe (the pair grid from given routes) suits a batch
+    whatever its routes are: every (pair, weight tile) workgroup looks at all
+    pairs, and each of an expert's 16-route tiles reads and quantises its rows
+    again, so the batch has to be small enough that a few busy experts cost no
+    more than on the route sort's chain.  Step, chain -> pair grid, us, random
+    routes and all rows on the same eight experts: E256 H2048 I512 5 rows 43 ->
+    35 and 31 -> 20, 24 rows 92 -> 85 and 33 -> 30; E128 H2048 I768 16 rows 83
+    -> 77 and 35 -> 29, 32 rows 108 -> 105 but 39 -> 46; E16 H1024 I256 32 rows
+    31 -> 22 and 31 -> 21 (half-width rows stay ahead up to 32 rows)."""
+    few = rows <= 16 or (rows <= 32 and (rows * top_k < num_experts or hidden <= 1024))
+    return (few and rows * top_k <= SORTLESS_PAIRS
+            and sortless_covers(rows, hidden, intermediate, top_k))
+
+
 def rows_in_view(x: torch.Tensor) -> bool:
     """Whether the rows span less than the 2 GiB that a kernel's buffer view
     of them covers (the route sort's chain reads rows of any stride)."""

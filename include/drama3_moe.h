@@ -455,8 +455,8 @@ int d3_decode_expert_gemm(int32_t mode, const uint8_t *w, const float *ws, int32
  * (three launches, no route sort): small_batch_moe
  * (src/drama3/kernels.py:325-357).  FC1 quantises the bf16 rows of its
  * routes while staging them and finds them in the ids (a workgroup per
- * (pair, weight tile) where there are fewer pairs than experts, else per
- * (expert, weight tile)), FC2 takes the SwiGLU requant in its prologue, then
+ * (pair, weight tile): each of an expert's 16-route tiles is the workgroup's
+ * of its first pair), FC2 takes the SwiGLU requant in its prologue, then
  * d3_weighted_combine.  Every expert contracts on the exact path.
  *   w13 / w2 fragment-major; x bf16 [rows, x_stride] (16-byte aligned rows);
  *   ids int32 or int64 [rows, top_k] (an expert may repeat in a row; pairs

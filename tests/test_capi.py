@@ -337,3 +337,17 @@ def test_decode_step_default_chains(slots, experts, sortless):
     else:
         with pytest.raises(ValueError):
             DecodeStep(slots, experts, 1024, 256, device="cpu", frontless=True)
+
+
+@pytest.mark.parametrize("rows,experts,hidden,inter,top_k,suited", [
+    (1, 256, 2048, 512, 8, True), (16, 256, 2048, 512, 8, True), (31, 256, 2048, 512, 8, True),
+    (32, 256, 2048, 512, 8, False), (16, 128, 2048, 768, 8, True), (17, 128, 2048, 768, 8, False),
+    (32, 16, 1024, 256, 8, True), (33, 16, 1024, 256, 8, False), (64, 256, 2048, 512, 2, False),
+    (200, 256, 2048, 512, 1, False), (256, 4, 1024, 256, 1, False), (5, 256, 4096, 512, 8, False)])
+def test_small_batch_route(rows, experts, hidden, inter, top_k, suited):
+    """Given routes skip the route sort only in batches so small that it pays
+    whatever the routes are: a busy expert's rows are read again by each of its
+    workgroups."""
+    from drama3_amd.pipeline import small_suited
+
+    assert small_suited(rows, experts, hidden, inter, top_k) == suited

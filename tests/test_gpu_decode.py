@@ -321,20 +321,24 @@ def test_standalone_entries_match_the_step(device):
 
 
 @pytest.mark.parametrize("ids_dtype", [torch.int32, torch.int64])
-@pytest.mark.parametrize("rows,experts,repeats", [(1, 256, False), (5, 256, True), (31, 256, False),
-                                                  (32, 256, False), (32, 128, False), (9, 16, False),
-                                                  (32, 16, True), (32, 4, True)])
-def test_small_moe_matches_sorted_chain(device, rows, experts, repeats, ids_dtype):
-    """The sortless chain from given ids (pair grid below one route per
-    expert, expert grid from there) against the sorted chain, bit for bit:
-    strided x rows, both id types, rows that repeat an expert (up to every
-    pair on one expert)."""
+@pytest.mark.parametrize("rows,experts,h,i,repeats", [
+    (1, 256, 1024, 256, False), (5, 256, 1024, 256, True), (31, 256, 1024, 256, False),
+    (32, 256, 1024, 256, False), (32, 128, 1024, 256, False), (9, 16, 1024, 256, False),
+    (32, 16, 1024, 256, True), (32, 4, 1024, 256, True),
+    # wide rows: the units of more than eight routes are staged in a second pass
+    (3, 40, 2048, 512, False), (12, 16, 2048, 512, False), (16, 9, 2048, 768, False),
+    (24, 40, 2048, 512, True), (32, 8, 2048, 768, False), (32, 5, 2048, 512, True)])
+def test_small_moe_matches_sorted_chain(device, rows, experts, h, i, repeats, ids_dtype):
+    """The sortless chain from given ids (the pair grid) against the sorted
+    chain, bit for bit: strided x rows, both id types, experts of one route, of
+    9 to 16 and of several route tiles, rows that repeat an expert (up to
+    nearly every pair on one expert)."""
     from drama3_amd.expert_weights import prepare_experts
     from drama3_amd.pipeline import MoEWorkspace, Shape
     from drama3_amd.workloads import make_experts
 
     gen = torch.Generator("cpu").manual_seed(31 * rows + experts)
-    h, i, top_k = 1024, 256, 8
+    top_k = 8
     weights = torch.rand((rows, top_k), generator=gen).to(device)
     if repeats:
         ids = torch.randint(0, experts, (rows, top_k), generator=gen)
