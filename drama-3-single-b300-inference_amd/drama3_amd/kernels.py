@@ -16,12 +16,9 @@ from . import _lib
 from ._lib import call, ptr
 from .pipeline import (WIDE_SORT_PAIRS, MoEWorkspace, Shape, by_pair_suited,
                        dtype_code, fragment_weights, grouped_supported, require_cuda,
-                       rows_in_view, small_suited, sortless_suited)
+                       routed_suited, rows_in_view, small_suited)
 
 TOP_K = 8
-# Most rows of routed_moe without a route sort (no expert has more routes than
-# rows, so every expert stays on the exact path).
-SORTLESS_ROWS = 64
 
 # Workspaces of the eager entry points, reused across calls with the same
 # shape, options, device and current stream (calls on one stream run in
@@ -314,8 +311,8 @@ def routed_moe(x, router, experts, decode=True, *, row_slots=None, padding_start
                                          padding_start=padding_start)
     if x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
-    if (rows <= SORTLESS_ROWS and sortless_suited(rows, e, h, i, TOP_K)
-            and fragment_weights(experts)):
+    # (at most 64 rows: no expert has more routes than the exact path takes)
+    if routed_suited(rows, e, h, i, TOP_K) and fragment_weights(experts):
         ws = _workspace(Shape(rows, e, h, i, TOP_K), x.device, sortless=True)
         return ws.forward(x, logits, experts, out=out)
     by_pair = by_pair_suited(rows, e, TOP_K) and grouped_supported(h, i)

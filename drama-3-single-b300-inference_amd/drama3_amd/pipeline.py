@@ -147,6 +147,25 @@ def small_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
             and sortless_covers(rows, hidden, intermediate, top_k))
 
 
+def routed_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
+                  top_k: int = 8) -> bool:
+    """Whether the front and the expert GEMMs without a route sort suit a
+    batch whatever its router says: fewer pairs than experts in up to 32 rows
+    (the pair grid, two route tiles per expert), or up to 64 rows of few enough
+    experts that the expert grid's FC1 is one round of resident workgroups.
+    Elsewhere the expert grid walks a busy expert's weight tiles once more per
+    16 routes.  Step, route sort -> expert grid, us, random routes / a router
+    biased by 0.75 of its logits' deviation / all rows on the same eight
+    experts: E16 H1024 I256 64 rows 37 -> 26, 42 -> 26, 43 -> 26; E128 H2048
+    I768 64 rows 118 -> 107, but 97 -> 132, 46 -> 267; E256 H2048 I512 48 rows
+    123 -> 116, 83 -> 137, 37 -> 254; E64 H2048 I768 9 rows 58 -> 58, 51 -> 56,
+    34 -> 45; pair grid, E256 24 rows 88 -> 82, 63 -> 62, 33 -> 33."""
+    pairs = rows * top_k
+    pair_grid = rows <= 32 and pairs <= SORTLESS_PAIRS and pairs < num_experts
+    one_round = rows <= 64 and num_experts <= 32 and num_experts * intermediate <= 16384
+    return (pair_grid or one_round) and sortless_covers(rows, hidden, intermediate, top_k)
+
+
 def rows_in_view(x: torch.Tensor) -> bool:
     """Whether the rows span less than the 2 GiB that a kernel's buffer view
     of them covers (the route sort's chain reads rows of any stride)."""

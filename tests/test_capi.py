@@ -351,3 +351,17 @@ def test_small_batch_route(rows, experts, hidden, inter, top_k, suited):
     from drama3_amd.pipeline import small_suited
 
     assert small_suited(rows, experts, hidden, inter, top_k) == suited
+
+
+@pytest.mark.parametrize("rows,experts,hidden,inter,suited", [
+    (1, 256, 2048, 512, True), (15, 128, 2048, 768, True), (16, 128, 2048, 768, False),
+    (31, 256, 2048, 512, True), (32, 256, 2048, 512, False), (64, 256, 2048, 512, False),
+    (64, 128, 2048, 768, False), (9, 64, 2048, 768, False), (33, 64, 1024, 256, False),
+    (64, 16, 1024, 256, True), (65, 16, 1024, 256, False), (64, 16, 2048, 768, True),
+    (17, 32, 2048, 768, False), (5, 256, 4096, 512, False)])
+def test_routed_route(rows, experts, hidden, inter, suited):
+    """Routes of a router skip the route sort only where that pays whatever the
+    router prefers."""
+    from drama3_amd.pipeline import routed_suited
+
+    assert routed_suited(rows, experts, hidden, inter) == suited

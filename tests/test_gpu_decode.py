@@ -399,3 +399,32 @@ def test_small_moe_rows_far_apart(device):
     far.copy_(x)
     got, expected = (small_batch_moe(t, ids, weights, packed) for t in (far, x))
     assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
+
+
+@pytest.mark.parametrize("experts,h,i,rows", [
+    (16, 1024, 256, (1, 2, 16, 17, 64)),    # expert grid (one row: pair grid)
+    (40, 2048, 768, (1, 4, 5, 33)),         # pair grid, then the sort
+    (272, 1024, 256, (16, 17, 32, 33))])    # pair grid of two route tiles, then the sort
+def test_routed_moe_small_batches_match_sorted_chain(device, experts, h, i, rows):
+    """routed_moe on prepared weights, at both sides of its rule, against the
+    front and the sorted chain, bit for bit: random routers, and all rows on
+    the same eight experts."""
+    from drama3_amd.expert_weights import prepare_experts
+    from drama3_amd.kernels import routed_moe
+    from drama3_amd.pipeline import MoEWorkspace, Shape
+    from drama3_amd.workloads import make_experts
+
+    gen = torch.Generator("cpu").manual_seed(experts)
+    packed = prepare_experts(make_experts(gen, experts, h, i).to(device))
+    for n in rows:
+        x = torch.randn((n, h), generator=gen).to(torch.bfloat16).to(device)
+        for hot in (False, True):
+            logits = torch.randn((n, experts), generator=gen)
+            if hot:
+                logits[:, 3:11] += 20
+            logits = logits.to(torch.bfloat16).to(device)
+            chain = MoEWorkspace(Shape(n, experts, h, i), device)
+            expected = chain.forward(x, logits, packed)
+            got = routed_moe(x, logits, packed)
+            torch.cuda.synchronize()
+            assert torch.equal(got.view(torch.int16), expected.view(torch.int16)), (n, hot)
