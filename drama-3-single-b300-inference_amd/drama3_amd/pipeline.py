@@ -102,6 +102,9 @@ def default_item_rows(rows: int, tile: int = SORT_TILE, num_experts: int | None 
 
 
 SORTLESS_PAIRS = 256  # most (row, rank) pairs of the expert GEMMs' pair grid
+# Most experts x intermediate columns whose FC1 expert grid (64 weight rows a
+# workgroup) is one round of resident workgroups (two on each of 256 CUs).
+ONE_ROUND_COLUMNS = 16384
 
 
 def sortless_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
@@ -113,12 +116,20 @@ def sortless_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
 
     Many experts with eight or more routes each, from more than 64 rows, are
     the sorted chain's: the sortless GEMMs then walk their weight tiles again
-    for experts beyond 16 routes (step, sortless -> sorted: E128 128 rows 144
-    -> 126 us, 256 rows 221 -> 140 us; E256 256 rows 160 us either way; E128
-    100 rows, 6 per expert, 112 against 122 us).  With few experts their
-    route slices run side by side instead (E16: 26 against 42 us)."""
+    for experts beyond 16 routes, unless their FC1 is one round of workgroups
+    (few experts: the route slices run side by side).  Step, sortless ->
+    sorted, us, random routers / routers biased by 0.75 of their logits'
+    deviation, all slots live: E128 H2048 I768 160 slots 165 -> 128 / 175 ->
+    115, 256 slots 213 -> 144 / 235 -> 142; E256 H2048 I512 256 slots 209 ->
+    164 / 359 -> 143; E64 H2048 I768 128 slots 110 -> 88 / 126 -> 90; one
+    round: E64 H1024 I256 128 slots 34 against 39 / 48 against 47; E16 H1024
+    I256 256 slots 38 against 54 / 46 against 54.  At exactly eight routes per
+    expert (E128 128 slots) random routers pay for the sort, 116 -> 127 (half
+    of the slots live 109 -> 120), where uneven ones gain more, 298 -> 117 (134
+    -> 96), and so do few live slots (4: 72 -> 44)."""
     pairs = rows * top_k
-    busy = rows > 64 and num_experts >= 64 and pairs >= 8 * num_experts
+    busy = (rows > 64 and num_experts >= 64 and pairs >= 8 * num_experts
+            and num_experts * intermediate > ONE_ROUND_COLUMNS)
     return (sortless_covers(rows, hidden, intermediate, top_k) and not busy
             and (pairs >= num_experts or pairs <= SORTLESS_PAIRS))
 
@@ -162,7 +173,8 @@ def routed_suited(rows: int, num_experts: int, hidden: int, intermediate: int,
     34 -> 45; pair grid, E256 24 rows 88 -> 82, 63 -> 62, 33 -> 33."""
     pairs = rows * top_k
     pair_grid = rows <= 32 and pairs <= SORTLESS_PAIRS and pairs < num_experts
-    one_round = rows <= 64 and num_experts <= 32 and num_experts * intermediate <= 16384
+    one_round = (rows <= 64 and num_experts <= 32
+                 and num_experts * intermediate <= ONE_ROUND_COLUMNS)
     return (pair_grid or one_round) and sortless_covers(rows, hidden, intermediate, top_k)
 
 

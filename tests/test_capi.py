@@ -322,7 +322,7 @@ def test_packed_operands_follow_their_source_tensor():
 
 @pytest.mark.parametrize("slots,experts,sortless",
                          [(64, 128, True), (128, 128, False), (256, 128, False), (256, 16, True),
-                          (16, 256, True), (64, 4096, False)])
+                          (72, 64, True), (256, 64, True), (16, 256, True), (64, 4096, False)])
 def test_decode_step_default_chains(slots, experts, sortless):
     """The chain a DecodeStep takes by default, and that asking for the
     three-launch step is answered alike whichever chain the default is: taken
