@@ -447,10 +447,13 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
     float as_prev = 0.0f;
 #pragma unroll
     for (int rt = 0; rt <= kRT; ++rt) {
-      if (kb + 1 < KB) {  // units rt (and, on the last route tile, the rest)
+      // Unit rt; units above kRT with the last route tile.  (Unit kRT too, and
+      // not after the last MFMAs: the step of E64 H2048 I768 131 rows 87 -> 97
+      // us, E16 H2048 I768 517 rows 69 -> 76.)
+      if (kb + 1 < KB) {
 #pragma unroll
         for (int u = 0; u < kUnits; ++u)
-          if (u == rt || (rt == kRT - 1 && u >= kRT)) issue_unit(kb + 1, u);
+          if (u == rt || (rt == kRT - 1 && u > kRT)) issue_unit(kb + 1, u);
       }
       float as = 0.0f;
       if (rt < kRT) {
@@ -669,10 +672,10 @@ __device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& ite
       float as_prev = 0.0f;
 #pragma unroll
       for (int rt = 0; rt <= kRT; ++rt) {
-        if (kb + 1 < KB) {  // units rt (and, on the last route tile, the rest)
+        if (kb + 1 < KB) {  // as in grouped_by_pair_kernel
 #pragma unroll
           for (int u = 0; u < kUnits; ++u) {
-            if (u != rt && !(rt == kRT - 1 && u >= kRT)) continue;
+            if (u != rt && !(rt == kRT - 1 && u > kRT)) continue;
             if (u < kStaged)
               staged[0][u] = view.load16(src[u] + (kb + 1) * kGroup);
             else
@@ -1029,5 +1032,3 @@ extern "C" int d3_grouped_fc1_swiglu_by_pair(const uint8_t* w13, const float* s1
   if (status != D3_OK) return status;
   D3_LAUNCHED("grouped_fc1_swiglu_by_pair");
 }
-
-
