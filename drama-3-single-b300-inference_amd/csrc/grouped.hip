@@ -73,11 +73,11 @@ constexpr int kGgXcds = 8;
 // (grouped_items_kernel, kSparse), if they fill a round of resident workgroups
 // (two per CU): below one round the launch is one prologue and K loop, 0.5 us
 // faster the other way (E16 H1024 I256, 140 rows).  Kernel trace, FC1 / FC2
-// us, dense -> sparse: E256 I512 3,000 rows (94 routes per expert) 119.5 / 95.7
-// -> 114.5 / 88.0, 3,300 rows (103) 123.3 / 98.5 -> 120.2 / 93.6, 3,600 rows
-// (113) 137.3 / 100.9 -> 138.5 / 98.7; E128 I768 1,500 rows (94) 96.6 / 64.3 ->
-// 92.0 / 62.0, 1,700 rows (106) 97.5 / 71.1 -> 98.1 / 71.5, 1,900 rows (119)
-// 99.7 / 71.6 -> 110.6 / 77.4.
+// us, dense -> sparse: E256 I512 3,000 rows (94 routes per expert) 113.5 / 92.1
+// -> 107.8 / 83.9, 3,300 rows (103) 126.6 / 94.5 -> 123.8 / 92.7, 3,600 rows
+// (113) 128.9 / 96.0 -> 132.7 / 99.1; E128 I768 1,500 rows (94) 96.9 / 63.0 ->
+// 88.0 / 55.5, 1,700 rows (106) 96.2 / 70.4 -> 95.9 / 70.2, 1,900 rows (119)
+// 97.0 / 71.9 -> 102.5 / 74.4.
 constexpr int kSparseRoutes = 104;
 constexpr int kResidentGroups = 512;
 constexpr int kStreamOutRoutes = 16384;  // FC2 launches up to this many item routes stream their rows
@@ -522,7 +522,8 @@ struct ItemLds {
 // for that many K blocks of weights; a block reloads the registers of the one
 // just multiplied (kSpread: of the one before, its loads between the MFMAs).
 // Activations take as many (one for kRT > 4, whose accumulators need the
-// registers).  K blocks in ascending order, one rescale per MFMA: the sums
+// registers).  kSparse: for items that stream an expert's weights alone.  K
+// blocks in ascending order, one rescale per MFMA: the sums
 // are the same in every body.
 template <int KB, int MODE, bool kPacked, bool kStreamOut, bool kSparse, int kRT, int kDepth>
 __device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& item, ItemLds<KB, MODE>& lds) {
@@ -531,8 +532,8 @@ __device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& ite
   constexpr int kStage = kR * kGgStride;
   constexpr int kD = kDepth < KB ? kDepth : KB;             // K blocks in flight
   constexpr int kA = kRT > 4 ? 1 : kD;                       // K blocks of activations in registers
-  // Contraction-sized items of dense batches: the next block's loads go out
-  // between the MFMAs.
+  // Contraction-sized items that share their expert's weights: the next
+  // block's loads go out between the MFMAs.
   constexpr bool kSpread = !kSparse && kRT > 4;
   constexpr int kStaged = kR * kGroup / (16 * kGgThreads);  // 16-byte copies per thread and K block
   static_assert(kStaged >= 1, "at least 32 routes: one copy per thread and K block");
@@ -578,8 +579,8 @@ __device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& ite
       const_cast<uint8_t*>(wexp), 0, static_cast<uint32_t>(n_rows) * K, 0x00020000);
   const uint32_t w_lane = kPacked ? lane * 16 : row16 * K + group * 16;
   int32x8 wf[kD][kGgWaveTiles];
-  // Sparse batches read the weights non-temporally (most experts have this
-  // item only); otherwise an expert's next item finds them in the L2.
+  // Read non-temporally where the expert most likely has this item only;
+  // otherwise its next item finds the weights in the L2.
   constexpr int kStreamed = kSparse && kPacked ? 2 : 0;
   auto load_tile = [&](int kb, int t) {
     const uint32_t base = static_cast<uint32_t>(tile_row(t)) * K;
@@ -747,28 +748,34 @@ __device__ __forceinline__ void item_body(const ItemArgs& a, const WorkItem& ite
 // The grouped GEMMs over sorted items.
 //
 // kSparse: batches of at most kSparseRoutes routes per expert on average.
-// They are bound by the weight stream, each expert's weights being read once,
-// by its one work item: registers go to weights in flight in every body, read
-// non-temporally.  Measured against a kernel of the 128-route body alone, one
-// cached K block in flight (E256 H2048 I512, FC1 / FC2 us, kernel trace, one
-// card): 131 rows (4 routes per expert) 104.8 / 61.8 -> 87.6 / 46.1 (6.1 / 6.0
-// TB/s), 517 rows of an uneven router 92.0 / 60.2 -> 84.1 / 48.4, 2048 rows
-// (64 per expert) 117.3 / 84.0 -> 106.6 / 78.6; non-temporal loads are half
-// of the gain.  Other depths (2 and 4 blocks for the 32-route body) are
+// They are bound by the weight stream, most experts' weights being read once,
+// by their one work item: registers go to weights in flight, read
+// non-temporally.  Items of more than 96 routes are the exception: there most
+// belong to an expert of several items, which share its weights in the L2, and
+// multiply as in a dense batch.  FC1 / FC2 us (kernel trace, one card) against
+// a kernel of the 128-route body alone, one cached K block in flight: E256
+// H2048 I512 131 rows (4 routes per expert) 104.6 / 59.6 -> 87.8 / 46.5 (6.1 /
+// 5.8 TB/s), 2,048 rows (64) 112.3 / 82.8 -> 99.0 / 72.6; routers biased by
+// 0.75 of their logits' deviation: 517 rows 90.9 / 59.4 -> 85.5 / 48.7, 2,048
+// rows 118.7 / 82.4 -> 118.4 / 78.5, 3,000 rows 126.1 / 99.9 -> 122.4 / 92.7,
+// E128 H2048 I768 1,500 rows 109.3 / 67.5 -> 95.4 / 68.3 (with the sparse loads
+// in the 128-route body too 128.0 / 81.1, 143.2 / 100.6 and 108.2 / 78.0 in
+// the last three).  Other depths (2 and 4 blocks for the 32-route body) are
 // within 1 us, 5 spills.
 //
 // Otherwise an expert has more than one item, which share its weights in the
-// L2 (cached loads; non-temporal 145 -> 157 us for FC1 at 4,096 rows), and the
-// matrix work of its full items wants the loads spread between the MFMAs; its
-// last item is often partial and takes a smaller body.  Against the 128-route
-// body for every item (same card, FC1 / FC2 us): 3,668 rows E128 I768 with the
-// shared expert 172.4 / 122.5 -> 161.6 / 115.1, 4,096 rows E256 I512 145.4 /
-// 119.5 -> 144.7 / 110.9, 2,500 rows E128 137.2 / 94.7 -> 131.3 / 90.7, 140
-// rows E16 H1024 I256 15.7 / 7.8 -> 13.8 / 6.5.  Bound: about half by waiting
-// for the K blocks' loads (one block ahead is what the accumulators leave),
-// the rest MFMAs and their rescale in turn.  64-route items at three waves per
-// SIMD were slower (165 -> 185 us: more weight traffic per MFMA), three weight
-// blocks for the 96-route body equal.
+// L2 (cached loads; non-temporal 160 -> 182 us for FC1 at 4,096 rows E256), and
+// the matrix work of its full items wants the loads spread between the MFMAs;
+// its last item is often partial and takes a smaller body.  Against the
+// 128-route body for every item (same card, FC1 / FC2 us, runs differ by 3):
+// 3,668 rows E128 I768 with the shared expert 173.8 / 117.2 -> 168.8 / 116.1,
+// 2,500 rows E128 120.0 / 88.4 -> 118.2 / 85.5, 3,600 rows E256 I512, biased
+// router 163.1 / 129.6 -> 150.3 / 117.3, 140 rows E16 H1024 I256 15.6 / 7.6 ->
+// 13.5 / 6.7; 4,096 rows E256 I512 156.7 / 127.6 and 159 / 127.5, no gain.
+// Bound: about half by waiting for the K blocks' loads (one block ahead is what
+// the accumulators leave), the rest MFMAs and their rescale in turn.  64-route
+// items at three waves per SIMD were slower (165 -> 185 us: more weight traffic
+// per MFMA), three weight blocks for the 96-route body equal.
 template <int KB, int MODE, bool kPacked, bool kStreamOut, bool kSparse>
 __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2))) void grouped_items_kernel(
     ItemArgs a) {
@@ -806,7 +813,7 @@ __global__ __launch_bounds__(kGgThreads) __attribute__((amdgpu_waves_per_eu(2)))
   else if (item.routes <= 96)
     item_body<KB, MODE, kPacked, kStreamOut, kSparse, 6, 2>(a, item, lds);
   else
-    item_body<KB, MODE, kPacked, kStreamOut, kSparse, 8, 2>(a, item, lds);
+    item_body<KB, MODE, kPacked, kStreamOut, false, 8, 2>(a, item, lds);
 }
 
 struct GroupedLaunch {
