@@ -164,7 +164,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   auto& route_pairs = lds.route_pairs;
   auto& route_slots = lds.route_slots;
   auto& chunk_counts = lds.chunk_counts;
-  int first_route = 16 * slice;  // this slice's (pair grid: this pair's) first route tile
+  const int first_route = 16 * slice;  // this slice's first route tile
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int row16 = lane & 15;
@@ -177,6 +177,7 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
   int expert = unit;
   uint32_t pair_ids[kPairGridPairs / kWave];
   uint64_t pair_hits[kPairGridPairs / kWave];
+  int rank = 0;  // of this pair among the expert's
   if constexpr (kPairGrid) {
     const uint32_t words = static_cast<uint32_t>(capacity * top_k * a.id_words);
     const BufferView id_view(a.ids, words * 4);
@@ -189,7 +190,6 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
     const int pairs = live_rows(a.row_count, capacity) * top_k;
     expert = __builtin_amdgcn_readfirstlane(static_cast<int>(own));
     if (unit >= pairs || expert < 0 || expert >= a.num_experts) return;  // uniform
-    int rank = 0;  // of this pair among the expert's
 #pragma unroll
     for (int c = 0; c < kPairGridPairs / kWave; ++c) {
       const int p = c * kWave + lane;
@@ -199,7 +199,6 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
       rank += __popcll(pair_hits[c] & mask);
     }
     if (rank % 16 != 0) return;  // uniform: an earlier pair's workgroup has this pair's route tile
-    first_route = rank;
   }
   const uint8_t* wexp = w + static_cast<size_t>(expert) * n_rows * K;
   const float* wsexp = ws + static_cast<size_t>(expert) * (n_rows / kGroup) * KB;
@@ -378,11 +377,12 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
     load_weights(first_tile, 0, kWholeFirst ? KB : kFirstHalf);
     load_scales(first_tile, 0, kWholeFirst ? KB : kFirstHalf);
     __builtin_amdgcn_sched_barrier(0);
+    // The list holds this workgroup's route tile only; the others are other pairs'.
     routes = 0;
 #pragma unroll
     for (int c = 0; c < kPairGridPairs / kWave; ++c) {
-      if (wave == 0 && ((pair_hits[c] >> lane) & 1ull)) {
-        const int r = routes + __popcll(pair_hits[c] & lanemask_lt());
+      const int r = routes + __popcll(pair_hits[c] & lanemask_lt()) - rank;
+      if (wave == 0 && ((pair_hits[c] >> lane) & 1ull) && r >= 0 && r < 16) {
         route_pairs[r] = c * kWave + lane;
         if constexpr (kFromX) route_slots[r] = (c * kWave + lane) / top_k;
       }
@@ -435,11 +435,12 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
     routes = chunk_base;
   }
   __syncthreads();
+  const bool exact = __builtin_amdgcn_readfirstlane(routes) <= exact_routes;
+  if constexpr (kPairGrid) routes = min(routes - rank, 16);
   routes = __builtin_amdgcn_readfirstlane(routes);
   // No route for this expert (or for this slice): the loads issued so far
   // are dropped.
   if (routes <= first_route) return;
-  const bool exact = routes <= exact_routes;
 
   // 4. Staging of one route tile (16 threads per route column), branch-free.
   const int stage_col = threadIdx.x >> 4;
@@ -704,7 +705,6 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
     floatx4 acc[RT];
     mma(acc);
     epilogue(acc, first_tile);
-    if constexpr (kPairGrid) return;  // further route tiles are other pairs'
     for (int m0 = first_route + 16 * slices; m0 < routes; m0 += 16 * slices) {
       __syncthreads();  // previous route tile fully consumed
       fetch_tile(m0);
@@ -751,13 +751,11 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2)
   decode_gemm_body<KB, RT, MODE, TILES, PASSES, kWholeFirst, true>(a, lds, expert, first_tile, slice, slices);
 }
 
-// The pair grid: workgroup -> (pair, weight tile).
+// The pair grid: block (weight tile, pair).
 template <int KB, int RT, int MODE>
 __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2))) void pair_gemm_kernel(DecodeArgs a) {
   __shared__ DecodeLds<KB, MODE> lds;
-  const int tiles = a.n_rows / (kGemmWaves * RT * 16);
-  const int unit = static_cast<int>(blockIdx.x) / tiles;
-  decode_gemm_body<KB, RT, MODE, 1, 1, false, true, true>(a, lds, unit, static_cast<int>(blockIdx.x) % tiles, 0, 1);
+  decode_gemm_body<KB, RT, MODE, 1, 1, false, true, true>(a, lds, blockIdx.y, blockIdx.x, 0, 1);
 }
 
 bool aligned(const void* p, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
@@ -851,7 +849,7 @@ void launch_decode(int num_experts, hipStream_t s, const DecodeArgs& a, bool by_
   const int tiles = a.n_rows / tile_rows_for(KB);
   if constexpr (MODE != 1) {
     if (MODE == 3 || by_pairs || pair_grid(num_experts, a.capacity, a.top_k)) {
-      hipLaunchKernelGGL((pair_gemm_kernel<KB, rt_for(KB), MODE>), dim3(a.capacity * a.top_k * tiles),
+      hipLaunchKernelGGL((pair_gemm_kernel<KB, rt_for(KB), MODE>), dim3(tiles, a.capacity * a.top_k),
                          dim3(kGemmThreads), 0, s, a);
       return;
     }
