@@ -62,6 +62,7 @@ struct DecodeArgs {
   // output, or none); the pair grid reads them as 32-bit words, id_words apart
   const int32_t* ids;
   int id_words;
+  int zero_skipped;  // pair grid, MODE 2: pairs with an id outside [0, num_experts) get zero rows
   const int32_t* row_count;
   // MODE 0: q rows and their scales; MODE 2: bf16 gate|up by pair
   const void* act;
@@ -189,7 +190,15 @@ __device__ __forceinline__ void decode_gemm_body(const DecodeArgs& a, DecodeLds<
     }
     const int pairs = live_rows(a.row_count, capacity) * top_k;
     expert = __builtin_amdgcn_readfirstlane(static_cast<int>(own));
-    if (unit >= pairs || expert < 0 || expert >= a.num_experts) return;  // uniform
+    if (unit >= pairs) return;  // uniform
+    if (__builtin_expect(expert < 0 || expert >= a.num_experts, 0)) {  // uniform: a skipped pair
+      if constexpr (MODE == 2) {
+        if (a.zero_skipped != 0 && threadIdx.x < kRowsPerGroup / 4)
+          *reinterpret_cast<float4*>(out_f32 + static_cast<size_t>(unit) * n_rows + first_tile * kRowsPerGroup +
+                                     threadIdx.x * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
+      return;
+    }
 #pragma unroll
     for (int c = 0; c < kPairGridPairs / kWave; ++c) {
       const int p = c * kWave + lane;
@@ -1364,6 +1373,7 @@ extern "C" int d3_small_moe(const uint8_t* w13, const float* s13, const uint8_t*
                              top_k, gate_up, nullptr, kPairGridPairs, nullptr, down, &fc2);
   if (status != D3_OK) return status;
   fc2.args.id_words = fc1.args.id_words;
+  fc2.args.zero_skipped = 1;
   fc2.by_pairs = true;
   hipStream_t s = as_stream(stream);
   launch_expert_gemm(fc1, s);

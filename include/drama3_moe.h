@@ -459,8 +459,9 @@ int d3_decode_expert_gemm(int32_t mode, const uint8_t *w, const float *ws, int32
  * of its first pair), FC2 takes the SwiGLU requant in its prologue, then
  * d3_weighted_combine.  Every expert contracts on the exact path.
  *   w13 / w2 fragment-major; x bf16 [rows, x_stride] (16-byte aligned rows);
- *   ids int32 or int64 [rows, top_k] (an expert may repeat in a row; pairs
- *   with an id outside [0, E) are skipped), weights bf16 or f32 [rows, top_k];
+ *   ids int32 or int64 (the low 32 bits) [rows, top_k]: an expert may repeat
+ *   in a row, and a pair with an id outside [0, E) adds a zero row;
+ *   weights bf16 or f32 [rows, top_k];
  *   gate_up bf16 [rows * top_k, 2I], down f32 [rows * top_k, H]: scratch;
  *   out bf16 [rows, H].  rows * top_k <= 256, top_k <= 8, H in {1024, 2048},
  *   I in {256, 512, 768, 1024}.

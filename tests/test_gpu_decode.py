@@ -428,3 +428,34 @@ def test_routed_moe_small_batches_match_sorted_chain(device, experts, h, i, rows
             got = routed_moe(x, logits, packed)
             torch.cuda.synchronize()
             assert torch.equal(got.view(torch.int16), expected.view(torch.int16)), (n, hot)
+
+
+@pytest.mark.parametrize("ids_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("h,i", [(1024, 256), (2048, 768)])
+def test_small_moe_pairs_without_expert(device, h, i, ids_dtype):
+    """Pairs whose id names no expert add nothing, whatever the scratch holds."""
+    from drama3_amd.expert_weights import prepare_experts
+    from drama3_amd.pipeline import MoEWorkspace, Shape
+    from drama3_amd.workloads import make_experts
+
+    gen = torch.Generator("cpu").manual_seed(43)
+    rows, experts, top_k = 6, 8, 8
+    packed = prepare_experts(make_experts(gen, experts, h, i).to(device))
+    ids = torch.stack([torch.randperm(experts, generator=gen)[:top_k] for _ in range(rows)])
+    weights = torch.rand((rows, top_k), generator=gen)
+    x = torch.randn((rows, h), generator=gen).to(torch.bfloat16).to(device)
+    holes = torch.zeros((rows, top_k), dtype=torch.bool)
+    holes[0, 0] = holes[1, 7] = holes[3, 2] = True
+    holes[4] = True  # a row without any expert
+    bad = torch.tensor([-1, experts, experts + 5, -2 ** 31] * rows * 2).view(rows, top_k)
+    ws = MoEWorkspace(Shape(rows, experts, h, i, top_k), device)
+    got, expected = (torch.empty((rows, h), dtype=torch.bfloat16, device=device) for _ in range(2))
+    ws.small_forward(x, ids.to(device, ids_dtype), torch.where(holes, 0.0, weights).to(device), packed,
+                     expected)
+    ws.gate_up.fill_(float("nan"))
+    ws.down.fill_(float("nan"))
+    ws.small_forward(x, torch.where(holes, bad, ids).to(device, ids_dtype), weights.to(device), packed, got)
+    torch.cuda.synchronize()
+    # a zero weight and a zero row both leave the fp32 sum as it is
+    assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
+    assert not got[4].any()
