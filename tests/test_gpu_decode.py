@@ -358,8 +358,10 @@ def test_small_moe_matches_sorted_chain(device, rows, experts, h, i, repeats, id
     assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
 
 
-@pytest.mark.parametrize("slots,live", [(1, 1), (16, 11), (31, 31), (32, 20)])
-def test_few_slots_match_sorted_chain(device, slots, live):
+@pytest.mark.parametrize("slots,live,e,h,i", [(1, 1, 272, 1024, 512), (16, 11, 272, 1024, 512),
+                                              (31, 31, 272, 1024, 512), (32, 20, 272, 1024, 512),
+                                              (16, 13, 136, 2048, 256)])
+def test_few_slots_match_sorted_chain(device, slots, live, e, h, i):
     """Fewer routes than experts: DecodeStep runs the pair grid after the
     front; every byte as the sorted chain's."""
     from drama3_amd.expert_weights import prepare_experts
@@ -367,7 +369,6 @@ def test_few_slots_match_sorted_chain(device, slots, live):
     from drama3_amd.workloads import make_experts
 
     gen = torch.Generator("cpu").manual_seed(slots)
-    e, h, i = 272, 1024, 512
     packed = prepare_experts(make_experts(gen, e, h, i).to(device))
     few = DecodeStep(slots, e, h, i, device=device)
     assert few.uses_sortless(packed) and not few.frontless
@@ -459,3 +460,33 @@ def test_small_moe_pairs_without_expert(device, h, i, ids_dtype):
     # a zero weight and a zero row both leave the fp32 sum as it is
     assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
     assert not got[4].any()
+
+
+@pytest.mark.parametrize("slots,live", [(128, 128), (128, 50), (256, 230)])
+def test_busy_slots_match_sortless_chain(device, slots, live):
+    """Eight and more routes per expert over many experts: by default the
+    sorted chain, every byte as the sortless one's and close to the oracle."""
+    from drama3_amd.expert_weights import prepare_experts
+    from drama3_amd.pipeline import DecodeStep
+    from drama3_amd.workloads import make_experts
+
+    gen = torch.Generator("cpu").manual_seed(slots + live)
+    e, h, i = 128, 1024, 256
+    experts_cpu = make_experts(gen, e, h, i)
+    packed = prepare_experts(experts_cpu.to(device))
+    chain = DecodeStep(slots, e, h, i, device=device)
+    assert not chain.uses_sortless(packed)
+    sortless = DecodeStep(slots, e, h, i, device=device, sortless=True)
+    occupancy = torch.zeros(slots, dtype=torch.uint8)
+    occupancy[torch.randperm(slots, generator=gen)[:live]] = 1
+    xs = torch.randn((slots, h), generator=gen).to(torch.bfloat16)
+    ls = torch.randn((slots, e), generator=gen).to(torch.bfloat16)
+    for step in (chain, sortless):
+        step(occupancy.to(device), xs.to(device), ls.to(device), packed)
+    torch.cuda.synchronize()
+    assert compare(sortless, chain, by_slot=True) == live
+    active, _ = om.compact_slots(occupancy.numpy())
+    weights, ids = om.route(np_f32(ls)[active])
+    assert np.bincount(ids.ravel()).max() <= 64  # the exact path in every item
+    expected = om.expert_ffn(np_bf16(xs)[active], ids, weights, oracle_weights(experts_cpu))
+    assert_bf16_close(np_bf16(chain.workspace.out)[:live], expected, **EXACT)

@@ -88,11 +88,14 @@ def test_dense_bf16_pairs_write_silu_mul(device, rows, pairs, n, k):
 
 @pytest.mark.parametrize("rows,e,h,i,si", [(48, 16, 1024, 256, 256), (300, 16, 1024, 256, 512),
                                            (64, 128, 2048, 768, 512),
+                                           # a decode bucket on the route sort's chain
+                                           (128, 128, 1024, 256, 256),
                                            # the reference model's layer (E256, I512, shared I512)
                                            (64, 256, 2048, 512, 512),
                                            # prefill-sized layers: tiled projections
                                            (2048, 256, 2048, 512, 512), (4096, 64, 1024, 256, 512)],
-                         ids=["r48_e16", "r300_e16", "r64_e128", "r64_reference_shape",
+                         ids=["r48_e16", "r300_e16", "r64_e128", "r128_e128",
+                              "r64_reference_shape",
                               "r2048_reference_shape", "r4096_e64"])
 def test_moe_layer_parts_and_combine(device, rows, e, h, i, si):
     from drama3_amd.kernels import combine_experts, combine_experts_add_norm
@@ -143,6 +146,36 @@ def test_moe_layer_parts_and_combine(device, rows, e, h, i, si):
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
     print(f"rows {rows} E {e} H {h} I {i} shared {si}: routed {stats}, "
           f"fused epilogue {layer._fused(experts, x, layer._views()[1])}", flush=True)
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+def test_moe_layer_busy_bucket_matches_sortless(device, rows):
+    """Decode buckets with eight and more routes per expert take the route
+    sort's chain by default: every byte as with the sortless chain and its
+    folded combine."""
+    from drama3_amd.moe_layer import MoELayer
+    from drama3_amd.pipeline import DecodeStep
+
+    gen = torch.Generator("cpu").manual_seed(rows)
+    e, h, i, si = 128, 1024, 256, 256
+    _, experts, projection, down = _weights(gen, e, h, i, si, device)
+    x = torch.randn((rows, h), generator=gen).to(torch.bfloat16).to(device)
+    residual = torch.randn((rows, h), generator=gen).to(torch.bfloat16).to(device)
+    norm_w = (torch.randn((h,), generator=gen) * 0.1).to(torch.bfloat16).to(device)
+    results = []
+    for sortless in (False, True):
+        layer = MoELayer(rows, e, h, i, si, device=device)
+        assert not layer.step.sortless
+        if sortless:
+            layer.step = DecodeStep(rows, e, h, i, device=device, sortless=True)
+        out = layer(x, projection, down, experts).clone()
+        res = residual.clone()
+        normed = layer.add_norm(x, projection, down, experts, res, norm_w, 1e-6).clone()
+        assert layer._fused(experts, x, layer._views()[1]) == sortless
+        results.append((out, res, normed))
+    torch.cuda.synchronize()
+    for a, b in zip(*results):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
 @pytest.mark.parametrize("logits_dtype,weights_dtype", [(torch.float32, torch.float32),
