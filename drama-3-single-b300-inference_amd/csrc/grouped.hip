@@ -14,21 +14,25 @@
 //     bodies that holds it (2, 4, 6 or 8 route tiles): at 8, 32 MFMAs per K
 //     block and 128 fp32 accumulators per lane; each B fragment read from
 //     LDS feeds four MFMAs.
-//   * Weights go straight from memory into MFMA fragments one K block ahead
-//     of the MFMAs (fragment-major layout: two 1 KiB contiguous loads per
-//     tile and K block; checkpoint layout: 16 rows x 64 bytes per load).
-//     Activation rows (gathered by route: FC1 reads token sorted_ids /
-//     top_k, FC2 the sorted row) are staged one K block ahead into a
-//     two-slot LDS ring (128 routes x 144-byte rows; the 16-byte pad keeps
-//     the 16 rows of each ds_read_b128 on distinct banks); their loads are
-//     issued before the weights', so waiting for them never waits for the
-//     weights.  In the contraction-sized bodies (6 and 8 route tiles) the
-//     next block's loads are issued in units spread over the current block's
-//     route tiles (one activation copy or one weight tile per route tile):
-//     issued in one block at its top they held the wave's MFMAs back while
-//     the memory pipeline drained (3 % slower per GEMM).  The smaller bodies
-//     keep two or three K blocks in flight in the registers they save.  One
-//     barrier per K block.
+//   * Weights go straight from memory into MFMA fragments (fragment-major
+//     layout: two 1 KiB contiguous loads per tile and K block; checkpoint
+//     layout: 16 rows x 64 bytes per load).  Activation rows (gathered by
+//     route: FC1 reads token sorted_ids / top_k, FC2 the sorted row) are
+//     staged through a two-slot LDS ring (128 routes x 144-byte rows; the
+//     16-byte pad keeps the 16 rows of each ds_read_b128 on distinct banks).
+//     One barrier per K block.
+//   * Order of the loads.  Contraction-sized bodies (6 and 8 route tiles; the
+//     6 of sparse launches excepted) and the by-pair kernel run one K block
+//     ahead, the next block's loads issued in units spread over the current
+//     block's route tiles, activation copies first, so that waiting for them
+//     never waits for the weights: issued in one block at its top they held
+//     the wave's MFMAs back while the memory pipeline drained (3 % slower per
+//     GEMM).  The other bodies keep two or three K blocks of weights in flight
+//     in the registers they save: route ids, half of these blocks, the
+//     activations, the rest, then each block's successor into the registers it
+//     leaves.  Up to 4 route tiles the activations take as many registers; at
+//     6 they load one block ahead, after that block's weights, whose arrival
+//     the store to LDS then waits for.
 //   * Measured per workgroup (per-workgroup timestamps, config-4 FC1): the
 //     prologue (item, route ids, scales, first blocks) and the epilogue
 //     cost a third of a workgroup's time; two resident workgroups per CU
@@ -988,8 +992,11 @@ extern "C" int d3_grouped_fc2(const uint8_t* w2, const float* s2, int32_t weight
                         reinterpret_cast<const int4*>(items), num_items, max_items, item_rows,
                         SharedItems{shared_w2, shared_s2, shared_rows, shared_act_row, shared_out_row},
                         nullptr, nullptr, down};
-  // The sorted rows hold the pairs and up to 15 padding rows per expert (at
-  // the 16-row sort tile; wider tiles and by-pair lists never come this low).
+  // The sorted rows hold the pairs and up to tile - 1 padding rows per expert:
+  // FC1's rule at the 16-row sort tile, but for the padding.  Wider tiles (64:
+  // from 57 routes per expert, 128: always) and by-pair lists leave FC2 on the
+  // dense bodies (a call of 517 rows E256 I512, sorted with 16 / 64 / 128 rows
+  // per tile: 173 / 179 / 179 us).
   g.sparse = act_rows - shared_rows <= static_cast<int64_t>(kSparseRoutes + 16) * num_experts;
   int status = check_grouped(g, num_experts, intermediate, act_rows, "grouped_fc2");
   if (status != D3_OK) return status;

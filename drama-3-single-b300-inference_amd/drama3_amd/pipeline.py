@@ -19,8 +19,10 @@ Step (one kernel each, all on the current stream):
     d3_expert_fc2_swiglu, and silu_mul_quant is not launched)
     weighted_combine sum_r w[t,r] y[t*K+r] -> bf16     (kernels.py:319-322,779)
 
-Decode step (``DecodeStep``, fragment-major weights, >= 1 route per expert): no
-route sort and no front launch.  ``decode_route_fc1`` routes (expert ranks
+Decode step (``DecodeStep``, fragment-major weights) of up to 64 slots with at
+least one route per expert, or of up to 256 where few experts' columns or less
+than eight routes per expert allow (``sortless_suited``): no route sort and no
+front launch.  ``decode_route_fc1`` routes (expert ranks
 from the logits), quantises and runs FC1 from the slots; ``decode_fc2``
 finds each expert's routes from the ids FC1 wrote and stores its down rows
 by slot pair (slot * top_k + rank); ``decode_route_combine`` recomputes the
@@ -744,13 +746,18 @@ class DecodeStep:
 
     Output row r belongs to slot ``active[r]`` for r < ``count``.
 
-    The sortless chain (``sortless``) normally starts with the front launch;
-    with ``frontless`` (default: whenever the sortless chain runs and the
-    inputs fit ``d3_decode_route_fc1``) the FC1 routes and quantises the
-    slots itself and the combine recomputes the routing weights, so the step
-    is three launches.  Same outputs (``out``, ``active``, ``count``,
-    workspace ``ids`` / ``weights`` / ``gate_up`` / ``down``); ``q`` and
-    ``x_scales`` are not written.
+    The chain depends on the shape (``sortless_suited``): the sortless one
+    (``sortless``), after the front launch with fewer routes than experts, or
+    the route sort's, the default from 65 slots with eight routes per expert
+    over many experts.  With ``frontless`` (default: whenever the sortless
+    chain runs, the slots' routes could reach every expert and the inputs fit
+    ``d3_decode_route_fc1``) the FC1 routes and quantises the slots itself and
+    the combine recomputes the routing weights, so the step is three launches.
+    ``out``, ``active``, ``count`` and the workspace's ``ids`` / ``weights`` are
+    the same on every chain.  ``gate_up`` / ``down`` rows are by pair on the
+    sortless chain (``down`` by slot pair when frontless), ``gate_up`` by sorted
+    row on the route sort's; ``q`` and ``x_scales`` are not written when
+    frontless.
     """
 
     def __init__(self, slots: int, num_experts: int, hidden: int, intermediate: int,

@@ -441,7 +441,8 @@ int d3_expert_fc2_swiglu(const uint8_t *w2, const float *s2, int32_t weight_layo
  * Values equal d3_expert_gemm's for the same pair.  Weights must be
  * fragment-major (d3_pack_expert_weights).  A workgroup of an expert with no
  * route reads half a weight tile before it knows, so this suits batches
- * whose routes cover most experts.  capacity <= 256, top_k <= 8; k in
+ * whose routes cover most experts; with fewer pairs than experts, at most
+ * 256, the grid is (pair, weight row tile) instead.  capacity <= 256, top_k <= 8; k in
  * {1024, 2048} (mode 0) or {256, 512, 768, 1024} (mode 2).
  */
 int d3_decode_expert_gemm(int32_t mode, const uint8_t *w, const float *ws, int32_t num_experts,
