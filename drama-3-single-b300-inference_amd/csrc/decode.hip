@@ -1164,11 +1164,11 @@ int check_ids_fc1(const uint8_t* w, const float* ws, int32_t num_experts, int32_
   D3_REQUIRE(ids_dtype == D3_DTYPE_I32 || ids_dtype == D3_DTYPE_I64, "small_moe: ids must be int32 or int64");
   D3_REQUIRE(num_experts >= 1 && n > 0 && k > 0 && n % kGroup == 0 && k % 256 == 0,
              "small_moe: N=%d must be a multiple of 128 and K=%d of 256", n, k);
-  D3_SUPPORTED(rows >= 1 && top_k >= 1 && top_k <= 8 && rows * top_k <= kPairGridPairs,
+  D3_SUPPORTED(rows >= 1 && rows <= kPairGridPairs && top_k >= 1 && top_k <= 8 && rows * top_k <= kPairGridPairs,
                "small_moe: rows %d x top_k %d (<= 8) above %d routes", rows, top_k, kPairGridPairs);
   D3_REQUIRE(x_stride >= k, "small_moe: row stride");
   D3_SUPPORTED(aligned(x, 16) && x_stride % 8 == 0, "small_moe: x rows must be 16-byte aligned");
-  D3_SUPPORTED(static_cast<int64_t>(rows) * x_stride * 2 < (int64_t{1} << 31), "small_moe: rows above 2 GiB");
+  D3_SUPPORTED(x_stride <= ((int64_t{1} << 30) - 1) / rows, "small_moe: rows above 2 GiB");
   D3_REQUIRE(aligned(w, 16) && aligned(gate_up, 16), "small_moe: alignment");
   const int kb = k / kGroup;
   D3_SUPPORTED(kb == 8 || kb == 16, "small_moe: K=%d not in the compiled set", k);

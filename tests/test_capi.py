@@ -215,6 +215,22 @@ def test_decode_gemm_contract(lib):
                   64, 16, None, None)
 
 
+def test_small_moe_contract(lib):
+    from drama3_amd import _lib
+
+    p = 256  # any aligned non-null address: every call below is rejected before a launch
+    call = [p, p, p, p, 16, 1024, 256, p, 1024, 4, p, _lib.DTYPE_I32, p, _lib.DTYPE_F32, 8, p, p, p, None]
+    for index, value, match in [(9, 33, "routes"), (9, 1 << 29, "routes"), (9, (1 << 29) + 1, "routes"),
+                                (14, 9, "routes"), (14, 0, "routes"), (8, 1016, "stride"),
+                                (8, 1028, "aligned"), (8, 1 << 28, "2 GiB"), (8, 1 << 62, "2 GiB"),
+                                (11, _lib.DTYPE_F32, "ids"), (13, _lib.DTYPE_I32, "weights"),
+                                (5, 768, "K=768"), (15, None, "null")]:
+        bad = list(call)
+        bad[index] = value
+        with pytest.raises(ValueError, match=match):
+            _lib.call("d3_small_moe", *bad)
+
+
 def test_route_fc1_and_combine_contract(lib):
     from drama3_amd import _lib
 
